@@ -122,12 +122,13 @@ int grm_hip_chunk_update_fwd_noalloc(const void* keys, const void* values, const
  *   forward as the op's aux); otherwise it is a workspace that the backward fills by
  *   running the forward again.
  * dkq_partial: float32 workspace [2, batch, ceil(value_dim / 16), seq_len, key_dim]
- *   (caller-provided).  The scalar kernel keeps per 16-column value tile partial sums of
- *   grad_keys and grad_queries there; the MFMA kernels for 16-bit inputs keep the adjoint
- *   dL/dM at every 64-token chunk end, [batch, ceil(seq_len / 64), value_dim, key_dim], at
- *   its front (they run when that fits, from about ten tokens on), followed, when the walk
- *   over the chunks runs in parts, by each part's adjoint at its start
- *   [batch, parts, value_dim, key_dim].
+ *   (caller-provided).  Both forms of the backward keep an adjoint dL/dM per 64-token
+ *   chunk, [batch, ceil(seq_len / 64), value_dim, key_dim], at its front (the MFMA kernels
+ *   for 16-bit inputs run when that fits, from about ten tokens on; the float32 kernels
+ *   need none for a single chunk).  The MFMA kernels' follow it, when the walk over the
+ *   chunks runs in parts, by each part's adjoint at its start
+ *   [batch, parts, value_dim, key_dim]; the float32 kernels', when several workgroups
+ *   share a chunk, by their partial sums of grad_keys and grad_queries.
  */
 int grm_hip_chunk_update_bwd(const void* grad_hidden, const void* grad_memory_out, const void* keys,
                              const void* values, const void* queries, const void* memory,

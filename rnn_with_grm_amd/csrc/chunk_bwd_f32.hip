@@ -1,0 +1,580 @@
+// Gradient of the chunked linear-memory update + query application in float32
+// arithmetic, gfx950: float32 inputs, and 16-bit inputs that the 16-bit MFMA
+// kernels of chunk_bwd.hip do not take (odd widths, unaligned rows, key_dim
+// above 128).
+//
+// Adjoint of  M_t = decay M_{t-1} + c v_t k_t^T,  h_t = M_t q_t   (c = (1-decay)/sqrt(d_k))
+// (reference grm/csrc/chunk_update.cu:137-278 and :588-716; CPU autograd in
+// grm_cuda.cpp:92-126).  Per 64-token chunk of L tokens, from the state M at its
+// start and the adjoint G at its end, with D[i][j] = decay^{i-j} (j <= i),
+// P = c (Q K^T) o D and dS = c (dH V^T) o D:
+//   dQ = decay^{i+1} dH M + dS K
+//   dK = dS^T Q + c decay^{L-1-j} V G
+//   dV = P^T dH + c decay^{L-1-j} K G^T
+//   G at the chunk's start = decay^L G + dH^T diag(decay^{i+1}) Q
+// Only the last line carries from chunk to chunk, and its second term does not
+// depend on G.  So three launches, each parallel over chunks or elements:
+//   bwd_outer_kernel  dH^T diag(decay^{i+1}) Q of every chunk
+//   bwd_carry_kernel  the recurrence over chunks, one thread per state element
+//   bwd_chunk_kernel  everything else, one workgroup per (sequence, chunk, share
+//                     of the value tiles), on float32 MFMA
+// With few chunks the value tiles of one chunk are shared by several workgroups
+// (`splits`), whose dQ and dK are partial sums that split_sum_kernel adds in order.
+//
+// What bounds it: float32 MFMA (16x16x4, 256 FLOP per CU and clock).  Every
+// operand comes from LDS as 16 bytes of a row or as four single elements of a
+// column, 64 bytes per clock and CU at most, half of what LDS gives; row strides
+// of 4 mod 64 elements keep both forms free of bank conflicts.
+//
+// Measured, forward and backward of 4 x 2000 float32 tokens, key_dim 64, value_dim
+// 512: 9.59 ms with a kernel that swept the tokens one by one (16 value rows per
+// wave, 128 waves on the chip), 120 us with these; error of the gradients against
+// 64 bits 7.1e-7 before, 2.6e-7 now.
+#include <stdint.h>
+
+#include <algorithm>
+
+#include "chunk_bwd.h"
+#include "grm_hip.h"
+#include "grm_hip_common.h"
+
+namespace grmhip {
+namespace {
+
+constexpr int GNT = 256;          // threads per workgroup
+constexpr int GVS = kGenDv + 4;   // LDS row stride of the V and dH tiles
+constexpr int GPS = BCT + 4;      // LDS row stride of P and dS
+constexpr int OUTER_V = 64;       // value rows per bwd_outer_kernel workgroup
+
+__device__ __forceinline__ f32x4 mfma4(f32x4 a, f32x4 b, f32x4 acc) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc, 0, 0, 0);
+  return acc;
+}
+
+// Four consecutive elements of an LDS row (reduction slots 4g + s of a 16-deep step).
+template <class E>
+__device__ __forceinline__ f32x4 lds_row4(const typename ET<E>::raw* p) {
+  f32x4 r;
+  if constexpr (sizeof(typename ET<E>::raw) == 2) {
+    const uint2 u = *reinterpret_cast<const uint2*>(p);
+    r[0] = ET<E>::to_f(static_cast<uint16_t>(u.x & 0xffffu));
+    r[1] = ET<E>::to_f(static_cast<uint16_t>(u.x >> 16));
+    r[2] = ET<E>::to_f(static_cast<uint16_t>(u.y & 0xffffu));
+    r[3] = ET<E>::to_f(static_cast<uint16_t>(u.y >> 16));
+  } else {
+    const float4 u = *reinterpret_cast<const float4*>(p);
+    r[0] = u.x; r[1] = u.y; r[2] = u.z; r[3] = u.w;
+  }
+  return r;
+}
+
+// Four elements of an LDS column, rows p, p + stride, ...
+template <class E>
+__device__ __forceinline__ f32x4 lds_col4(const typename ET<E>::raw* p, int stride) {
+  f32x4 r;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) r[s] = ET<E>::to_f(p[s * stride]);
+  return r;
+}
+
+// Four consecutive output elements at element `el` (`left` of them inside the row).
+template <class E>
+__device__ __forceinline__ void out4(__amdgpu_buffer_rsrc_t r, int el, int left, bool vec, f32x4 v) {
+  constexpr int ES = static_cast<int>(sizeof(typename ET<E>::raw));
+  if (vec) {
+    buf_store4<E>(r, left > 0 ? el * ES : kBufOOB, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) buf_store1<E>(r, i < left ? (el + i) * ES : kBufOOB, v[i]);
+  }
+}
+
+__device__ __forceinline__ float ld_mem(__amdgpu_buffer_rsrc_t r, int el, bool f32, bool ok, F32) {
+  (void)f32;
+  return buf_load1<F32>(r, ok ? el * 4 : kBufOOB);
+}
+template <class E>
+__device__ __forceinline__ float ld_mem(__amdgpu_buffer_rsrc_t r, int el, bool f32, bool ok, E) {
+  return f32 ? buf_load1<F32>(r, ok ? el * 4 : kBufOOB) : ET<E>::to_f(buf_load1<E>(r, ok ? el * 2 : kBufOOB));
+}
+
+template <class E>
+__device__ __forceinline__ float ld_state(const void* p, int64_t i, bool f32) {
+  return f32 ? static_cast<const float*>(p)[i] : ET<E>::to_f(static_cast<const typename ET<E>::raw*>(p)[i]);
+}
+
+// dH^T diag(decay^{i+1}) Q of one chunk: workgroup (sequence, chunk, 64 value
+// rows), wave w rows [16w, +16), every key column.  Operands straight from
+// global memory (64-byte row pieces per 16 lanes, each used once per wave).
+// One chunk (n_chunks == 1): grad_memory itself, decay^L grad_memory_out added.
+template <class E, int DKP>
+__global__ __launch_bounds__(GNT) void bwd_outer_kernel(const BwdGenArgs a) {
+  using raw = typename ET<E>::raw;
+  constexpr int ES = static_cast<int>(sizeof(raw));
+  constexpr int KT = DKP / 16;
+  __shared__ float pw[BCT + 1];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, g = lane >> 4, n = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int dk = a.dk, dv = a.dv;
+  const int vtiles = (dv + OUTER_V - 1) / OUTER_V;
+  const int vt = static_cast<int>(blockIdx.x % static_cast<unsigned>(vtiles));
+  const int64_t bc = blockIdx.x / static_cast<unsigned>(vtiles);
+  const int ch = static_cast<int>(bc % a.n_chunks);
+  const int64_t b = bc / a.n_chunks;
+  const int64_t t0 = static_cast<int64_t>(ch) * BCT;
+  const int L = ch == a.n_chunks - 1 ? static_cast<int>(a.T - t0) : BCT;
+  if (tid <= BCT) pw[tid] = a.pw[tid];
+  __syncthreads();
+  const __amdgpu_buffer_rsrc_t rq =
+      make_rsrc(static_cast<const raw*>(a.queries) + (b * a.T + t0) * dk, static_cast<uint32_t>(L * dk * ES));
+  const __amdgpu_buffer_rsrc_t rh =
+      make_rsrc(static_cast<const raw*>(a.dh) + (b * a.T + t0) * dv, static_cast<uint32_t>(L * dv * ES));
+  const int v = vt * OUTER_V + 16 * w + n;
+  float h[4][4];
+#pragma unroll
+  for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int i = 16 * ib + 4 * g + s;
+      h[ib][s] = ET<E>::to_f(buf_load1<E>(rh, v < dv ? (i * dv + v) * ES : kBufOOB));
+    }
+  f32x4 acc[KT];
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+    const int k = 16 * kt + n;
+    float q[4][4];
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        q[ib][s] = ET<E>::to_f(buf_load1<E>(rq, k < dk ? ((16 * ib + 4 * g + s) * dk + k) * ES : kBufOOB));
+    if (kt == 0) {
+#pragma unroll
+      for (int ib = 0; ib < 4; ++ib)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) h[ib][s] *= pw[16 * ib + 4 * g + s + 1];
+    }
+    acc[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib)
+      acc[kt] = mfma4(f32x4{q[ib][0], q[ib][1], q[ib][2], q[ib][3]}, f32x4{h[ib][0], h[ib][1], h[ib][2], h[ib][3]},
+                      acc[kt]);
+  }
+  if (v >= dv) return;
+  if (a.n_chunks == 1) {
+    const bool f32m = a.mem_f32 != 0;
+    const float decay_L = pw[L];
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int k = 16 * kt + 4 * g + r;
+        if (k >= dk) continue;
+        const int64_t i = (b * dv + v) * dk + k;
+        const float y = fmaf(decay_L, ld_state<E>(a.dmo, i, f32m), acc[kt][r]);
+        if (f32m) static_cast<float*>(a.dm_out)[i] = y;
+        else static_cast<raw*>(a.dm_out)[i] = ET<E>::from_f(y);
+      }
+    return;
+  }
+  const __amdgpu_buffer_rsrc_t ro = make_rsrc(a.gbuf + ((b * a.n_chunks + ch) * dv + vt * OUTER_V) * dk,
+                                              static_cast<uint32_t>(min(OUTER_V, dv - vt * OUTER_V) * dk * 4));
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+    const int k = 16 * kt + 4 * g;
+    out4<F32>(ro, (16 * w + n) * dk + k, dk - k, a.vec_k != 0, acc[kt]);
+  }
+}
+
+// Slot ch := decay^{L_ch} G + slot ch, G the value of slot ch + 1 (grad_memory_out
+// for the last chunk): slot ch then holds the adjoint at chunk ch's start, and
+// chunk 0's goes to grad_memory.  One thread per state element, eight loads ahead.
+template <class E>
+__global__ __launch_bounds__(GNT) void bwd_carry_kernel(const BwdGenArgs a) {
+  constexpr int AHEAD = 8;
+  const int64_t plane = static_cast<int64_t>(a.dv) * a.dk;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * GNT + threadIdx.x;
+  if (i >= a.batch * plane) return;
+  const int64_t b = i / plane;
+  float* slot = a.gbuf + b * a.n_chunks * plane + (i - b * plane);
+  const bool f32m = a.mem_f32 != 0;
+  float x = ld_state<E>(a.dmo, i, f32m);
+  const float decay_c = a.pw[BCT];
+  const float decay_last = a.pw[static_cast<int>(a.T - static_cast<int64_t>(a.n_chunks - 1) * BCT)];
+  float buf[AHEAD];
+#pragma unroll
+  for (int j = 0; j < AHEAD; ++j) {
+    const int ch = a.n_chunks - 1 - j;
+    buf[j] = ch >= 0 ? slot[ch * plane] : 0.f;
+  }
+  for (int top = a.n_chunks - 1; top >= 0; top -= AHEAD) {
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) {
+      const int ch = top - j;
+      if (ch < 0) break;
+      x = fmaf(ch == a.n_chunks - 1 ? decay_last : decay_c, x, buf[j]);
+      if (ch > 0) slot[ch * plane] = x;
+      const int next = ch - AHEAD;
+      buf[j] = next >= 0 ? slot[next * plane] : 0.f;
+    }
+  }
+  if (f32m) static_cast<float*>(a.dm_out)[i] = x;
+  else static_cast<typename ET<E>::raw*>(a.dm_out)[i] = ET<E>::from_f(x);
+}
+
+template <class E, int DKP>
+struct GenShape {
+  using raw = typename ET<E>::raw;
+  static constexpr int KS = DKP + 4;  // LDS row stride of K, Q (input type) and of M, G (float32)
+  static constexpr int KT = DKP / 16;
+  static constexpr int KQ_LOADS = BCT * DKP / GNT;
+  static constexpr int V_LOADS = BCT * kGenDv / GNT;
+  static constexpr int M_LOADS = kGenDv * DKP / GNT;
+  static constexpr size_t kq_bytes = 2ull * BCT * KS * sizeof(raw);
+  static constexpr size_t vh_bytes = 2ull * BCT * GVS * sizeof(raw);
+  static constexpr size_t mg_bytes = 2ull * kGenDv * KS * 4;
+  static constexpr size_t p_bytes = static_cast<size_t>(BCT) * GPS * 4;
+  // P (before the first value tile) and dS (after the last) share the value tiles' region.
+  static constexpr size_t tile_bytes = vh_bytes + mg_bytes > p_bytes ? vh_bytes + mg_bytes : p_bytes;
+  static constexpr size_t lds_bytes = kq_bytes + tile_bytes + (BCT + 1) * 4;
+  static_assert(lds_bytes <= 160 * 1024, "one workgroup's tiles fit the CU");
+  static_assert(kq_bytes % 16 == 0 && vh_bytes % 16 == 0 && tile_bytes % 16 == 0, "16-byte regions");
+};
+
+// The gradients of one chunk from its starting state and the adjoint at its end,
+// over value tiles [split * tiles_per_split, +tiles_per_split).  Wave w owns tokens
+// [16w, +16) of every product; lane (g, n) of an accumulator holds four
+// consecutive key (or value) columns 4g + r of token n.
+template <class E, int DKP>
+__global__ __launch_bounds__(GNT) void bwd_chunk_kernel(const BwdGenArgs a) {
+  using S = GenShape<E, DKP>;
+  using raw = typename ET<E>::raw;
+  constexpr int ES = static_cast<int>(sizeof(raw));
+  constexpr int KS = S::KS, KT = S::KT;
+  extern __shared__ __align__(16) unsigned char smem[];
+  raw* Ks = reinterpret_cast<raw*>(smem);  // [BCT][KS]
+  raw* Qs = Ks + BCT * KS;                 // [BCT][KS]
+  unsigned char* tile = smem + S::kq_bytes;
+  raw* Vs = reinterpret_cast<raw*>(tile);  // [BCT][GVS] value tile columns
+  raw* Hs = Vs + BCT * GVS;                // [BCT][GVS] grad_hidden tile columns
+  float* Ms = reinterpret_cast<float*>(tile + S::vh_bytes);  // [kGenDv][KS] the chunk's starting state
+  float* Gs = Ms + kGenDv * KS;                              // [kGenDv][KS] adjoint at the chunk's end
+  float* Ps = reinterpret_cast<float*>(tile);                // [BCT][GPS] P, then dS
+  float* pw = reinterpret_cast<float*>(tile + S::tile_bytes);
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, g = lane >> 4, n = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int split = static_cast<int>(blockIdx.x % static_cast<unsigned>(a.splits));
+  const int64_t bc = blockIdx.x / static_cast<unsigned>(a.splits);
+  const int ch = static_cast<int>(bc % a.n_chunks);
+  const int64_t b = bc / a.n_chunks;
+  const int dk = a.dk, dv = a.dv;
+  const int64_t t0 = static_cast<int64_t>(ch) * BCT;
+  const int L = ch == a.n_chunks - 1 ? static_cast<int>(a.T - t0) : BCT;
+  const float c = a.c;
+  const bool f32m = a.mem_f32 != 0;
+  const int64_t mem_b = f32m ? 4 : ES;
+  const int vt_begin = split * a.tiles_per_split;
+  const int vt_end = min(vt_begin + a.tiles_per_split, (dv + kGenDv - 1) / kGenDv);
+
+  if (tid <= BCT) pw[tid] = a.pw[tid];
+  {
+    const __amdgpu_buffer_rsrc_t rk =
+        make_rsrc(static_cast<const raw*>(a.keys) + (b * a.T + t0) * dk, static_cast<uint32_t>(L * dk * ES));
+    const __amdgpu_buffer_rsrc_t rq =
+        make_rsrc(static_cast<const raw*>(a.queries) + (b * a.T + t0) * dk, static_cast<uint32_t>(L * dk * ES));
+    constexpr int STEP = S::KQ_LOADS < 16 ? S::KQ_LOADS : 16;
+#pragma unroll 1
+    for (int u0 = 0; u0 < S::KQ_LOADS; u0 += STEP) {
+      raw kx[STEP], qx[STEP];
+#pragma unroll
+      for (int u = 0; u < STEP; ++u) {
+        const int l = tid + GNT * (u0 + u), row = l / DKP, col = l % DKP;
+        const int off = col < dk ? (row * dk + col) * ES : kBufOOB;
+        kx[u] = buf_load1<E>(rk, off);
+        qx[u] = buf_load1<E>(rq, off);
+      }
+#pragma unroll
+      for (int u = 0; u < STEP; ++u) {
+        const int l = tid + GNT * (u0 + u), row = l / DKP, col = l % DKP;
+        Ks[row * KS + col] = kx[u];
+        Qs[row * KS + col] = qx[u];
+      }
+    }
+  }
+
+  const unsigned char* msrc =
+      ch == 0 ? static_cast<const unsigned char*>(a.memory) + b * dv * dk * mem_b
+              : reinterpret_cast<const unsigned char*>(a.states + (b * a.n_chunks + ch - 1) * dv * dk);
+  const unsigned char* gsrc =
+      ch == a.n_chunks - 1 ? static_cast<const unsigned char*>(a.dmo) + b * dv * dk * mem_b
+                           : reinterpret_cast<const unsigned char*>(a.gbuf + (b * a.n_chunks + ch + 1) * dv * dk);
+  const bool m32 = ch != 0 || f32m, g32 = ch != a.n_chunks - 1 || f32m;
+  const __amdgpu_buffer_rsrc_t rv =
+      make_rsrc(static_cast<const raw*>(a.values) + (b * a.T + t0) * dv, static_cast<uint32_t>(L * dv * ES));
+  const __amdgpu_buffer_rsrc_t rh =
+      make_rsrc(static_cast<const raw*>(a.dh) + (b * a.T + t0) * dv, static_cast<uint32_t>(L * dv * ES));
+  struct Stage {
+    raw v[S::V_LOADS], h[S::V_LOADS];
+    float m[S::M_LOADS], gg[S::M_LOADS];
+  };
+  auto load_vtile = [&](int vt, Stage& sg) {
+    const int v0 = vt * kGenDv;
+#pragma unroll
+    for (int u = 0; u < S::V_LOADS; ++u) {
+      const int l = tid + GNT * u, row = l / kGenDv, col = v0 + l % kGenDv;
+      const int off = col < dv ? (row * dv + col) * ES : kBufOOB;
+      sg.v[u] = buf_load1<E>(rv, off);
+      sg.h[u] = buf_load1<E>(rh, off);
+    }
+    const int rows = min(kGenDv, dv - v0);
+    const int mb = m32 ? 4 : ES, gb = g32 ? 4 : ES;
+    const __amdgpu_buffer_rsrc_t rm =
+        make_rsrc(msrc + static_cast<int64_t>(v0) * dk * mb, static_cast<uint32_t>(rows * dk * mb));
+    const __amdgpu_buffer_rsrc_t rg =
+        make_rsrc(gsrc + static_cast<int64_t>(v0) * dk * gb, static_cast<uint32_t>(rows * dk * gb));
+#pragma unroll
+    for (int u = 0; u < S::M_LOADS; ++u) {
+      const int l = tid + GNT * u, row = l / DKP, col = l % DKP;
+      sg.m[u] = ld_mem(rm, row * dk + col, m32, col < dk, E());
+      sg.gg[u] = ld_mem(rg, row * dk + col, g32, col < dk, E());
+    }
+  };
+  auto store_vtile = [&](const Stage& sg) {
+#pragma unroll
+    for (int u = 0; u < S::V_LOADS; ++u) {
+      const int l = tid + GNT * u, o = (l / kGenDv) * GVS + l % kGenDv;
+      Vs[o] = sg.v[u];
+      Hs[o] = sg.h[u];
+    }
+#pragma unroll
+    for (int u = 0; u < S::M_LOADS; ++u) {
+      const int l = tid + GNT * u, o = (l / DKP) * KS + l % DKP;
+      Ms[o] = sg.m[u];
+      Gs[o] = sg.gg[u];
+    }
+  };
+  Stage stage;
+  load_vtile(vt_begin, stage);
+  __syncthreads();  // K, Q, pw
+
+  // c decay^{i-j} x for this lane's row i = 16w + n and keys j = 16 jb + 4g + r, zero right of the diagonal
+  const int jrow = 16 * w + n;
+  auto causal4 = [&](int jb, f32x4 x) {
+    f32x4 y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int j = 16 * jb + 4 * g + r;
+      y[r] = j <= jrow ? x[r] * (c * pw[max(jrow - j, 0)]) : 0.f;
+    }
+    return y;
+  };
+  const float sq = pw[jrow + 1];
+  const float wl = (jrow < L) ? c * pw[max(L - 1 - jrow, 0)] : 0.f;
+
+  // ---- P rows of query block w, then this wave's columns of P
+  f32x4 pT[4];
+  {
+    f32x4 s[4];
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb) s[jb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int kk = 0; kk < KT; ++kk) {
+      const f32x4 qf = lds_row4<E>(Qs + jrow * KS + 16 * kk + 4 * g);
+#pragma unroll
+      for (int jb = 0; jb < 4; ++jb)
+        if (jb <= w) s[jb] = mfma4(lds_row4<E>(Ks + (16 * jb + n) * KS + 16 * kk + 4 * g), qf, s[jb]);
+    }
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb)
+      *reinterpret_cast<float4*>(Ps + jrow * GPS + 16 * jb + 4 * g) =
+          __builtin_bit_cast(float4, causal4(jb, s[jb]));
+    __syncthreads();
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib) pT[ib] = lds_col4<F32>(Ps + (16 * ib + 4 * g) * GPS + jrow, GPS);
+    __syncthreads();  // P read: the region takes the value tiles
+  }
+
+  f32x4 dsacc[4], dq[KT], dkk[KT];
+#pragma unroll
+  for (int jb = 0; jb < 4; ++jb) dsacc[jb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) dq[kt] = dkk[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const __amdgpu_buffer_rsrc_t rdv =
+      make_rsrc(static_cast<raw*>(a.dv_out) + (b * a.T + t0) * dv, static_cast<uint32_t>(L * dv * ES));
+  for (int vt = vt_begin; vt < vt_end; ++vt) {
+    store_vtile(stage);
+    if (vt + 1 < vt_end) load_vtile(vt + 1, stage);
+    __syncthreads();  // value tile in LDS
+#pragma unroll
+    for (int cc = 0; cc < kGenDv / 16; ++cc) {
+      const f32x4 hf = lds_row4<E>(Hs + jrow * GVS + 16 * cc + 4 * g);
+      const f32x4 vf = lds_row4<E>(Vs + jrow * GVS + 16 * cc + 4 * g);
+      // dS rows of block w
+#pragma unroll
+      for (int jb = 0; jb < 4; ++jb)
+        if (jb <= w) dsacc[jb] = mfma4(lds_row4<E>(Vs + (16 * jb + n) * GVS + 16 * cc + 4 * g), hf, dsacc[jb]);
+      // dQ (sum_v dH[i][v] M[v][k]) and dK (sum_v G[v][k] V[j][v])
+#pragma unroll
+      for (int kt = 0; kt < KT; ++kt) {
+        const int o = (16 * cc + 4 * g) * KS + 16 * kt + n;
+        dq[kt] = mfma4(lds_col4<F32>(Ms + o, KS), hf, dq[kt]);
+        dkk[kt] = mfma4(lds_col4<F32>(Gs + o, KS), vf, dkk[kt]);
+      }
+    }
+    // dV rows of block w: c decay^{L-1-j} sum_k G[v][k] K[j][k] + sum_i dH[i][v] P[i][j]
+    f32x4 dvv[kGenDv / 16];
+#pragma unroll
+    for (int vb = 0; vb < kGenDv / 16; ++vb) dvv[vb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int kk = 0; kk < KT; ++kk) {
+      const f32x4 kf = lds_row4<E>(Ks + jrow * KS + 16 * kk + 4 * g);
+#pragma unroll
+      for (int vb = 0; vb < kGenDv / 16; ++vb)
+        dvv[vb] = mfma4(lds_row4<F32>(Gs + (16 * vb + n) * KS + 16 * kk + 4 * g), kf, dvv[vb]);
+    }
+#pragma unroll
+    for (int vb = 0; vb < kGenDv / 16; ++vb) {
+      f32x4 acc = dvv[vb] * wl;
+#pragma unroll
+      for (int ib = 0; ib < 4; ++ib)
+        if (ib >= w) acc = mfma4(lds_col4<E>(Hs + (16 * ib + 4 * g) * GVS + 16 * vb + n, GVS), pT[ib], acc);
+      const int v = vt * kGenDv + 16 * vb + 4 * g;
+      out4<E>(rdv, jrow * dv + v, dv - v, a.vec_v != 0, acc);
+    }
+    __syncthreads();  // every read of this tile done
+  }
+
+  // ---- dS complete.  dQ takes this wave's rows from registers (the accumulator
+  // layout is the operand layout), dK this wave's columns through LDS.
+#pragma unroll
+  for (int jb = 0; jb < 4; ++jb) {
+    dsacc[jb] = causal4(jb, dsacc[jb]);
+    *reinterpret_cast<float4*>(Ps + jrow * GPS + 16 * jb + 4 * g) = __builtin_bit_cast(float4, dsacc[jb]);
+  }
+  __syncthreads();
+  f32x4 dsT[4];
+#pragma unroll
+  for (int ib = 0; ib < 4; ++ib) dsT[ib] = lds_col4<F32>(Ps + (16 * ib + 4 * g) * GPS + jrow, GPS);
+  const bool partial = a.splits > 1;
+  const int64_t prow = ((b * a.splits + split) * a.T + t0) * dk;
+  const __amdgpu_buffer_rsrc_t rqo =
+      partial ? make_rsrc(a.part_q + prow, static_cast<uint32_t>(L * dk * 4))
+              : make_rsrc(static_cast<raw*>(a.dq_out) + (b * a.T + t0) * dk, static_cast<uint32_t>(L * dk * ES));
+  const __amdgpu_buffer_rsrc_t rko =
+      partial ? make_rsrc(a.part_k + prow, static_cast<uint32_t>(L * dk * 4))
+              : make_rsrc(static_cast<raw*>(a.dk_out) + (b * a.T + t0) * dk, static_cast<uint32_t>(L * dk * ES));
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+    f32x4 aq = dq[kt] * sq, ak = dkk[kt] * wl;
+#pragma unroll
+    for (int xb = 0; xb < 4; ++xb) {
+      const int o = (16 * xb + 4 * g) * KS + 16 * kt + n;
+      if (xb <= w) aq = mfma4(lds_col4<E>(Ks + o, KS), dsacc[xb], aq);
+      if (xb >= w) ak = mfma4(lds_col4<E>(Qs + o, KS), dsT[xb], ak);
+    }
+    const int k = 16 * kt + 4 * g;
+    if (partial) {
+      out4<F32>(rqo, jrow * dk + k, dk - k, a.vec_k != 0, aq);
+      out4<F32>(rko, jrow * dk + k, dk - k, a.vec_k != 0, ak);
+    } else {
+      out4<E>(rqo, jrow * dk + k, dk - k, a.vec_k != 0, aq);
+      out4<E>(rko, jrow * dk + k, dk - k, a.vec_k != 0, ak);
+    }
+  }
+}
+
+// out[b, t, k] = sum over splits of part[b, split, t, k], splits in order;
+// blockIdx.y 0: grad_keys, 1: grad_queries.
+template <class E>
+__global__ __launch_bounds__(GNT) void split_sum_kernel(const BwdGenArgs a) {
+  const float* part = blockIdx.y == 0 ? a.part_k : a.part_q;
+  void* out = blockIdx.y == 0 ? a.dk_out : a.dq_out;
+  const int64_t plane = a.T * a.dk, total = a.batch * plane;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * GNT + threadIdx.x; i < total;
+       i += static_cast<int64_t>(gridDim.x) * GNT) {
+    const int64_t b = i / plane;
+    const float* p = part + b * a.splits * plane + (i - b * plane);
+    float s = p[0];
+    for (int x = 1; x < a.splits; ++x) s += p[x * plane];
+    static_cast<typename ET<E>::raw*>(out)[i] = ET<E>::from_f(s);
+  }
+}
+
+template <class E, int DKP>
+int launch_gen(const BwdGenArgs& a, hipStream_t s) {
+  using S = GenShape<E, DKP>;
+  if (S::lds_bytes > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_chunk_kernel<E, DKP>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             static_cast<int>(S::lds_bytes));
+    if (e != hipSuccess) {
+      set_error("chunk_update_bwd: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+      return static_cast<int>(e);
+    }
+  }
+  const int64_t bc = a.batch * a.n_chunks;
+  hipLaunchKernelGGL((bwd_outer_kernel<E, DKP>), dim3(static_cast<unsigned>(bc * ((a.dv + OUTER_V - 1) / OUTER_V))),
+                     dim3(GNT), 0, s, a);
+  int rc = check_launch("chunk_update_bwd(outer)");
+  if (rc != GRM_HIP_OK) return rc;
+  if (a.n_chunks > 1) {
+    const int64_t n = a.batch * a.dv * a.dk;
+    hipLaunchKernelGGL(bwd_carry_kernel<E>, dim3(static_cast<unsigned>((n + GNT - 1) / GNT)), dim3(GNT), 0, s, a);
+    rc = check_launch("chunk_update_bwd(carry)");
+    if (rc != GRM_HIP_OK) return rc;
+  }
+  hipLaunchKernelGGL((bwd_chunk_kernel<E, DKP>), dim3(static_cast<unsigned>(bc * a.splits)), dim3(GNT), S::lds_bytes, s,
+                     a);
+  rc = check_launch("chunk_update_bwd(gradients)");
+  if (rc != GRM_HIP_OK || a.splits == 1) return rc;
+  const int64_t want = (a.batch * a.T * a.dk + GNT - 1) / GNT;
+  hipLaunchKernelGGL(split_sum_kernel<E>, dim3(static_cast<unsigned>(std::min<int64_t>(want, 4096)), 2), dim3(GNT), 0,
+                     s, a);
+  return check_launch("chunk_update_bwd(split sum)");
+}
+
+template <class E>
+int launch_gen_width(const BwdGenArgs& a, hipStream_t s) {
+  if (a.dk <= 32) return launch_gen<E, 32>(a, s);
+  if (a.dk <= 64) return launch_gen<E, 64>(a, s);
+  if (a.dk <= 128) return launch_gen<E, 128>(a, s);
+  if constexpr (sizeof(typename ET<E>::raw) == 2) return launch_gen<E, 256>(a, s);
+  set_error("chunk_update_bwd: key_dim %d exceeds 128 for float32", a.dk);
+  return GRM_HIP_EUNSUPPORTED;
+}
+
+}  // namespace
+
+int launch_bwd_gen(BwdGenArgs a, int in_dtype, float* ws, int64_t floats, hipStream_t s) {
+  const int64_t vtiles = (a.dv + kGenDv - 1) / kGenDv;
+  const int64_t adj = a.n_chunks > 1 ? a.batch * a.n_chunks * static_cast<int64_t>(a.dv) * a.dk : 0;
+  // Enough workgroups for two per CU, at least two value tiles each (a split
+  // repeats the chunk's P and its dS products, worth about one tile's work), and
+  // the partial sums within the workspace.
+  const int64_t bc = a.batch * a.n_chunks;
+  int64_t splits = std::max<int64_t>(1, std::min<int64_t>((512 + bc - 1) / bc, vtiles / 2));
+  const int64_t rows = a.batch * a.T * a.dk;
+  while (splits > 1 && adj + 2 * splits * rows > floats) --splits;
+  const int64_t per = (vtiles + splits - 1) / splits;
+  a.tiles_per_split = static_cast<int>(per);
+  a.splits = static_cast<int>((vtiles + per - 1) / per);
+  if (adj > floats || std::min<int64_t>(a.T, BCT) * a.dv * 4 > INT32_MAX || bc * a.splits > INT32_MAX || bc * ((a.dv + OUTER_V - 1) / OUTER_V) > INT32_MAX ||
+      (a.batch * a.dv * a.dk + GNT - 1) / GNT > INT32_MAX) {
+    set_error("chunk_update_bwd: problem too large for one launch");
+    return GRM_HIP_EINVAL;
+  }
+  a.gbuf = ws;
+  a.part_k = ws + adj;
+  a.part_q = ws + adj + a.splits * rows;
+  switch (in_dtype) {
+    case GRM_HIP_F32: return launch_gen_width<F32>(a, s);
+    case GRM_HIP_F16: return launch_gen_width<F16>(a, s);
+    default: return launch_gen_width<BF16>(a, s);
+  }
+}
+
+}  // namespace grmhip

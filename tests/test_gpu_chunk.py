@@ -395,6 +395,41 @@ def test_mfma_backward_parts(dev, monkeypatch, B, T, K, H, mem_dtype):
             assert float((x - y).abs().max()) <= 1e-5 * scale, name
 
 
+@pytest.mark.parametrize("dtype,mem_dtype,shift,B,T,K,H", [
+    (torch.float32, torch.float32, 0, 1, 1, 8, 16), (torch.float32, torch.float32, 0, 2, 64, 16, 31),
+    (torch.float32, torch.float32, 0, 2, 65, 25, 40), (torch.float32, torch.float32, 0, 1, 64, 64, 512),
+    (torch.float32, torch.float32, 0, 3, 700, 33, 96), (torch.float32, torch.float32, 0, 1, 130, 128, 257),
+    (torch.float32, torch.float32, 1, 2, 129, 64, 64), (torch.bfloat16, torch.float32, 1, 2, 129, 64, 64),
+    (torch.bfloat16, torch.bfloat16, 0, 2, 3, 25, 33), (torch.float16, torch.float32, 0, 2, 700, 25, 100),
+    (torch.bfloat16, torch.float32, 0, 1, 150, 200, 48), (torch.float16, torch.float16, 0, 1, 70, 256, 20)])
+def test_float32_backward(dev, dtype, mem_dtype, shift, B, T, K, H):
+    """The chunk-parallel float32 backward against the double-precision oracle: one token, one full
+    chunk, ragged last chunks, key widths on both sides of each padded width, value widths that are
+    no multiple of the 32-column tile, chunks shared by several workgroups (512 values, few chunks),
+    eleven chunks of carried adjoint (700 tokens), rows that start one element past an aligned
+    address (shift), and the 16-bit inputs that the 16-bit kernels refuse.  float32: 1e-5 (rtol and
+    atol) per element, the bar of test_chunk_backward."""
+    k, v, q, m = make_case(B, T, K, H, dtype, mem_dtype, seed=T + K)
+    g = torch.Generator().manual_seed(9)
+    dh = torch.randn(B, T, H, generator=g).to(dtype)
+    dm = torch.randn(B, H, K, generator=g).to(mem_dtype)
+
+    def place(t):
+        flat = torch.empty(t.numel() + shift, dtype=t.dtype, device=dev)[shift:]
+        return flat.copy_(t.flatten()).view(t.shape)
+
+    print(f"float32 backward {dtype} B={B} T={T} K={K} H={H} shift {shift}", flush=True)
+    got = capi.chunk_update_bwd(*[place(t) for t in (dh, dm, k, v, q, m)], 0.97)
+    torch.cuda.synchronize()
+    ref = orc.chunk_update_bwd(dh.double().numpy(), dm.double().numpy(), k.double().numpy(), v.double().numpy(),
+                               q.double().numpy(), m.double().numpy(), 0.97)
+    for name, x, r in zip(("grad_keys", "grad_values", "grad_queries", "grad_memory"), got, ref):
+        if x.dtype == torch.float32:
+            np.testing.assert_allclose(x.double().cpu().numpy(), r, rtol=1e-5, atol=1e-5, err_msg=name)
+        else:
+            close_elementwise(name, x, r)
+
+
 def test_autograd_through_cuda_ops(dev):
     """cuda_chunk_update under autograd matches the fallback's autograd (the
     reference's check, examples/test_grm.py:72-113)."""
