@@ -37,6 +37,7 @@ constexpr int64_t kMaxSegments = 16384;
 constexpr int AP_THREADS = 256;      // apply kernel: 4 waves
 constexpr int AP_V = kScaledTile;    // value rows per workgroup
 constexpr int AP_N = 64;             // (q, r) pairs per tile
+constexpr int kLdsApplyPairs = 256;  // see launch_scaled_rows
 
 struct RetrieveArgs {
   const void* mem;
@@ -65,11 +66,11 @@ struct RetrieveArgs {
   int32_t* tile_base;
   int tb_max;
   int tile_pairs;
-  // Gate-weighted, row-scaled 16-bit output (retrieve_fuse): out holds float16
-  // rows of g * M q scaled by 2^sh per (pair, 128-value tile), scales[pair,
-  // tile] = 2^-sh.  nullptr: the plain [pairs, dv] output of gather_apply.
-  const float* gates;  // [batch, n_index]
+  // Row-scaled 16-bit output (retrieve_fuse): out holds float16 rows of M q
+  // scaled by 2^sh per (pair, 128-value tile), scales[pair, tile] = 2^-sh, 0 for
+  // a pair without a row.  nullptr: the plain [pairs, dv] output of gather_apply.
   float* scales;       // [batch, n_index, v_tiles]
+  int mean_pairs;  // pairs per segment, evenly spread
   int out_row;         // elements per output row (dv; dk for the queries' gradient)
 };
 
@@ -135,8 +136,9 @@ __device__ __forceinline__ int nth_set_bit(uint64_t mask, int r) {
 }
 
 // A row whose index is outside [0, segments): zeros, and one count.  Called
-// by every lane of a wave together (bad: this lane's pair i is invalid).  With
-// 16-byte rows the wave writes several whole rows per store instruction,
+// by every lane of a wave together (bad: this lane's pair i is invalid).  Scaled
+// rows only get the scale 0, which fuse_scaled_kernel takes as an absent row.
+// With 16-byte rows the wave writes several whole rows per store instruction,
 // coalesced (the first segments' short windows can leave most of a pair chunk
 // empty); otherwise one row after another, consecutive lanes on consecutive
 // elements.
@@ -147,6 +149,11 @@ __device__ __forceinline__ void zero_rows_wave(const RetrieveArgs& a, int64_t b,
   const int lane = threadIdx.x & 63;
   if (mask != 0u && lane == 0 && a.bad != nullptr) atomicAdd(a.bad, static_cast<int>(__popcll(mask)));
   if (mask == 0u) return;
+  if (a.scales != nullptr) {
+    if (bad)
+      for (int t = 0; t < a.v_tiles; ++t) a.scales[(b * a.n_index + i) * a.v_tiles + t] = 0.f;
+    return;
+  }
   const int64_t row_bytes = static_cast<int64_t>(a.out_row) * sizeof(raw);
   if (row_bytes % 16 == 0 && reinterpret_cast<uintptr_t>(a.out) % 16 == 0) {
     // Whole rows in 16-byte pieces: lpr lanes per row, 64 / lpr rows per store
@@ -162,8 +169,6 @@ __device__ __forceinline__ void zero_rows_wave(const RetrieveArgs& a, int64_t b,
       if (r < m) {
         uint4* ob = reinterpret_cast<uint4*>(static_cast<raw*>(a.out) + (b * a.n_index + row) * a.out_row);
         for (int p = lane % lpr; p < pieces; p += lpr) ob[p] = uint4{0u, 0u, 0u, 0u};
-        if (a.scales != nullptr)
-          for (int t = lane % lpr; t < a.v_tiles; t += lpr) a.scales[(b * a.n_index + row) * a.v_tiles + t] = 0.f;
       }
     }
     return;
@@ -174,8 +179,6 @@ __device__ __forceinline__ void zero_rows_wave(const RetrieveArgs& a, int64_t b,
     const int64_t row = __shfl(i, l, 64);
     typename ET<EM>::raw* ob = static_cast<typename ET<EM>::raw*>(a.out) + (b * a.n_index + row) * a.out_row;
     for (int h = lane; h < a.out_row; h += 64) ob[h] = ET<EM>::from_f(0.f);
-    if (a.scales != nullptr)
-      for (int t = lane; t < a.v_tiles; t += 64) a.scales[(b * a.n_index + row) * a.v_tiles + t] = 0.f;
   }
 }
 
@@ -207,12 +210,32 @@ __global__ __launch_bounds__(BK_THREADS) void bucket_kernel(const RetrieveArgs a
 }
 
 // The same sort over many workgroups per sequence (three launches): counts per
-// pair group, per-(group, segment) bases, then the scatter.  Group c holds the
-// blocks of BK_THREADS pairs c, c + bk_chunks, c + 2 bk_chunks, ... (about
-// BK_ITEMS pairs): strided rather than contiguous, so that the empty slots of
-// the first segments' short windows, which can fill most of the first 16384
-// pairs, are zeroed by every group instead of one or two.  The order of pairs
-// inside a segment does not change any result.
+// pair group, per-(group, segment) bases, then the scatter.  The order of pairs
+// inside a segment does not change any result, but it decides which query rows
+// are read together.
+// Scaled rows: group c holds consecutive blocks of BK_THREADS pairs, so that a
+// segment's list follows the queries (in steps of a group) and workgroups on
+// different segments sweep them together (16 x 65536 queries over 512 states, with
+// the gates moved to the fusion: 3.60 -> 3.49 ms).
+// Plain rows: group c holds the blocks c, c + bk_chunks, c + 2 bk_chunks, ...:
+// the empty slots of the first segments' short windows, which can fill most of
+// the first 16384 pairs, are then zeroed by every group instead of one or two.
+struct PairBlocks {
+  int64_t first, end, step;
+  __device__ PairBlocks(const RetrieveArgs& a, int64_t group, int64_t n_blocks) {
+    if (a.scales != nullptr) {
+      const int64_t per = (n_blocks + a.bk_chunks - 1) / a.bk_chunks;
+      first = group * per;
+      end = min_i64(first + per, n_blocks);
+      step = 1;
+    } else {
+      first = group;
+      end = n_blocks;
+      step = a.bk_chunks;
+    }
+  }
+};
+
 template <class EM>
 __global__ __launch_bounds__(BK_THREADS) void bucket_count_kernel(const RetrieveArgs a) {
   extern __shared__ int hist[];  // [segments]
@@ -223,7 +246,8 @@ __global__ __launch_bounds__(BK_THREADS) void bucket_count_kernel(const Retrieve
   const int64_t* ib = a.idx + b * n;
   for (int64_t s = tid; s < S; s += BK_THREADS) hist[s] = 0;
   __syncthreads();
-  for (int64_t blk = chunk; blk < n_blocks; blk += a.bk_chunks) {  // uniform trip count: whole waves zero rows
+  const PairBlocks pb(a, chunk, n_blocks);
+  for (int64_t blk = pb.first; blk < pb.end; blk += pb.step) {  // uniform trip count: whole waves zero rows
     const int64_t i = blk * BK_THREADS + tid;
     const int64_t s = i < n ? ib[i] : 0;
     const bool valid = s >= 0 && s < S;
@@ -269,7 +293,8 @@ __global__ __launch_bounds__(BK_THREADS) void bucket_scatter_kernel(const Retrie
   for (int64_t s = tid; s < S; s += BK_THREADS) cur[s] = pc[s];
   __syncthreads();
   int32_t* lb = a.list + b * n;
-  for (int64_t blk = chunk; blk < n_blocks; blk += a.bk_chunks) {  // the count kernel's pair group
+  const PairBlocks pb(a, chunk, n_blocks);
+  for (int64_t blk = pb.first; blk < pb.end; blk += pb.step) {  // the count kernel's pair group
     const int64_t i = blk * BK_THREADS + tid;
     if (i >= n) continue;
     const int64_t s = ib[i];
@@ -665,9 +690,6 @@ __global__ __launch_bounds__(AP_THREADS) void apply_mfma16_kernel(const Retrieve
     const int pid_cur = pid_l;
     const bool more = p0 + AP_N < p_end;
     const int pid_next = (more && lane < p_end - p0 - AP_N) ? lb[p0 + AP_N + lane] : -1;
-    // The gate of this lane's pair, loaded while the tile's products run.
-    float gate_cur = 0.f;
-    if constexpr (SCALED) gate_cur = pid_cur >= 0 ? a.gates[b * a.n_index + pid_cur] : 0.f;
     if (!split) {
       split = true;
 #pragma unroll
@@ -726,10 +748,9 @@ __global__ __launch_bounds__(AP_THREADS) void apply_mfma16_kernel(const Retrieve
       const int pid = __shfl(pid_cur, p, 64);
       if constexpr (SCALED) {
         // The 32 lanes of one half-wave hold pair p's 128 values of this tile:
-        // scale the gate-weighted row so its largest magnitude lies in
-        // [2^14, 2^15) and store it as float16 with the inverse power of two.
-        const float gp = __shfl(gate_cur, p, 64);
-        const f32x4 val = *reinterpret_cast<const f32x4*>(Os + p * OS + v) * gp;
+        // scale the row so its largest magnitude lies in [2^14, 2^15) and store it
+        // as float16 with the inverse power of two.
+        const f32x4 val = *reinterpret_cast<const f32x4*>(Os + p * OS + v);
         float m = fmaxf(fmaxf(fabsf(val[0]), fabsf(val[1])), fmaxf(fabsf(val[2]), fabsf(val[3])));
         // maximum over the 32 lanes of the half-wave without LDS: quad swaps, the
         // half-row and row mirrors (DPP), then the 16-lane row swap
@@ -856,10 +877,12 @@ int dispatch_q(const RetrieveArgs& a, int q_dtype, hipStream_t s) {
 
 // ---------------------------------------------------------------------------
 // Residual + LayerNorm over the scaled rows of retrieve_fuse:
-//   out[t] = LN(h[t] + sum_r scales[t, r, c / 128] * rows[t, r, c])
+//   out[t] = LN(h[t] + sum_r gates[t, r] scales[t, r, c / 128] * rows[t, r, c])
 // h and out in E, the LayerNorm weight and bias in float32,
-// with r in order 0 .. R-1 (the gates are already in the rows), a two-pass
-// mean / variance in fp32.  lpr lanes share a row, each covering NV groups of
+// with r in order 0 .. R-1 (gates null: already in the rows; scale 0: no row), a
+// two-pass mean / variance in fp32.  The gates are read here, in order, rather than
+// where the rows are made, one scattered 4-byte read per pair (165 us of 2.4 ms at
+// 16 x 65536 queries with 16 routes).  lpr lanes share a row, each covering NV groups of
 // 8 consecutive columns (16-byte float16 loads of the rows).
 
 template <class E>
@@ -898,6 +921,7 @@ __global__ __launch_bounds__(256) void fuse_scaled_kernel(const FuseScaledArgs a
   using raw = typename ET<E>::raw;
   const int tid = threadIdx.x;
   const int sub = tid & (lpr - 1);
+  const int lane = tid & 63, per = min(lpr, AP_V / 8);  // lanes on one tile of a row (or the row)
   const WaveRows wr = wave_rows(static_cast<int64_t>(blockIdx.x) * (256 / lpr), lpr, a.n_rows);
   const bool live = wr.row < a.n_rows;
   const int H = a.hidden;
@@ -906,6 +930,7 @@ __global__ __launch_bounds__(256) void fuse_scaled_kernel(const FuseScaledArgs a
   const __amdgpu_buffer_rsrc_t rh = wave_rows_rsrc(a.h, wr, hb);
   const __amdgpu_buffer_rsrc_t rrow = wave_rows_rsrc(a.rows, wr, rowb);
   const float* sc = a.scales + rr * a.routes * a.v_tiles;
+  const float* ga = a.gates != nullptr ? a.gates + rr * a.routes : nullptr;
   float x[NV][8];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
@@ -917,13 +942,31 @@ __global__ __launch_bounds__(256) void fuse_scaled_kernel(const FuseScaledArgs a
 #pragma unroll
     for (int e = 0; e < 8; ++e) r[e] = 0.f;
     const int tile = c / AP_V;
-#pragma unroll 4
-    for (int j = 0; j < a.routes; ++j) {
-      const float sj = in ? sc[j * a.v_tiles + tile] : 0.f;
+    if (ga == nullptr && a.routes == 1) {  // the window retrieval's sums: always there
+      const float s0 = in ? sc[tile] : 0.f;
       float rv[8];
-      load8<F16>(rrow, in ? wr.local * rowb + (j * H + c) * 2 : kBufOOB, rv);
+      load8<F16>(rrow, in ? wr.local * rowb + c * 2 : kBufOOB, rv);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) r[e] = fmaf(sj, rv[e], r[e]);
+      for (int e = 0; e < 8; ++e) r[e] = fmaf(s0, rv[e], r[e]);
+    } else
+    // Scale and gate of 16 routes at a time (fewer with short rows), one per lane of
+    // the lanes on one tile; rows without a scale are not read.
+    for (int j0 = 0; j0 < a.routes; j0 += per) {
+      const int jl = j0 + (lane & (per - 1));
+      const bool have = live && tile < a.v_tiles && jl < a.routes;  // also on lanes past the row's end
+      const float sl = have ? sc[jl * a.v_tiles + tile] : 0.f;
+      const float gl = have && ga != nullptr ? ga[jl] : 1.f;
+      const float cl = sl != 0.f ? sl * gl : 0.f;
+      const uint64_t rows_there = __ballot(sl != 0.f);
+#pragma unroll 4
+      for (int t = 0; t < min(per, a.routes - j0); ++t) {
+        const int src = (lane & ~(per - 1)) + t;
+        const float cj = __shfl(cl, src, 64);
+        float rv[8];
+        load8<F16>(rrow, in && ((rows_there >> src) & 1) ? wr.local * rowb + ((j0 + t) * H + c) * 2 : kBufOOB, rv);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r[e] = fmaf(cj, rv[e], r[e]);
+      }
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[v][e] = c < H ? hv[e] + r[e] : 0.f;
@@ -1002,6 +1045,234 @@ int fuse_scaled(const FuseScaledArgs& a, int h_dtype, hipStream_t s) {
 
 namespace {
 
+// Many pairs per state, for the scaled rows of retrieve_fuse: the state's MFMA
+// operands in LDS, the pairs in registers.  Eight waves stage one 16 NI-row value
+// tile of the segment's state as NPART exact 16-bit parts in fragment order (1 KB
+// per fragment, read back without bank conflicts), then each wave takes 64 pairs
+// at a time on its own, with no barrier: an A fragment read from LDS serves four
+// MFMAs, and a lane ends with all values of four pairs (a quarter of each row), so
+// the gate, the row's scale and the 16-bit rows come straight from the
+// accumulators.  Row m = 4 g' + r of fragment i stands for value 32 (i >> 1) + 8 g' +
+// 4 (i & 1) + r: lane (g, n)'s accumulators of fragments 2p and 2p + 1 are then the
+// eight consecutive values 32 p + 8 g .. + 7 of pair n, one 16-byte store, and the four
+// lanes of a pair write 64 consecutive bytes.  The same products in the same order
+// as apply_mfma16_kernel, so the same bits.
+//
+// That kernel holds 32 rows per wave and passes every 64-pair output tile through
+// LDS with two barriers and eight dependent scale-and-store rounds per wave, which
+// cost more than its memory traffic.  16 x 65536 queries, 16 of 512 states of
+// 128 x 128: 3.4 ms there, 2.2 ms here.  What bounds it now: the 256-byte query rows
+// read and the rows written, both scattered, about 11 GB through the L2 misses at
+// 4.8 TB/s (a 1 GiB copy reaches 5.2); without the row stores 1.0 ms less, with 32
+// or 64 pairs per wave and step within 4%.
+constexpr int AL_THREADS = 512;
+constexpr int AL_WAVES = AL_THREADS / 64;
+constexpr int AL_NJ = 3;             // 16-pair columns per wave and step
+constexpr int AL_PAIRS = 16 * AL_NJ;  // pairs per wave and step
+
+template <class EL, class EQ, int DKP, class EF, int NPART, int NI>
+__global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const RetrieveArgs a) {
+  using rawl = typename ET<EL>::raw;
+  using rawf = typename ET<EF>::raw;
+  constexpr int NSTEP = DKP / 32;
+  constexpr int FRAGS = NSTEP * NI;  // fragments per part
+  static_assert(std::is_same_v<EQ, EF>, "the query's bits are the MFMA operand");
+  extern __shared__ __align__(16) unsigned char al_smem[];
+  Frag8<EF>* As = reinterpret_cast<Frag8<EF>*>(al_smem);  // [NPART][NSTEP][NI][64]
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, g = lane >> 4, n = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t vt = blockIdx.x % a.v_tiles;
+  const int64_t tile = blockIdx.x / a.v_tiles;
+  const int64_t b = blockIdx.y;
+  if (tile >= a.n_tiles[b]) return;
+  const int4 te = a.tiles[b * a.tb_max + tile];
+  const int p_end = te.z;
+  const int dk = a.dk, dv = a.dv;
+  const int v0 = static_cast<int>(vt) * AP_V;
+  const uint32_t index_bytes = static_cast<uint32_t>(a.n_index) * 4;
+  const __amdgpu_buffer_rsrc_t rl = make_rsrc(a.list + b * a.n_index, index_bytes);
+  const __amdgpu_buffer_rsrc_t rout =
+      make_rsrc(static_cast<const uint16_t*>(a.out) + b * a.n_index * dv, static_cast<uint32_t>(a.n_index * dv * 2));
+  const __amdgpu_buffer_rsrc_t rscale =
+      make_rsrc(a.scales + b * a.n_index * a.v_tiles, static_cast<uint32_t>(a.n_index * a.v_tiles * 4));
+  auto load_id = [&](int p) {  // -1 past the tile
+    const int id = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rl, p + lane < p_end ? (p + lane) * 4 : kBufOOB, 0, 0));
+    return p + lane < p_end ? id : -1;
+  };
+
+  // Pair ids (one per lane) of this wave's first 64 pairs, ids of the next.
+  int p0 = te.y + AL_PAIRS * w;
+  int pid = load_id(p0), pid_next = load_id(p0 + AL_PAIRS * AL_WAVES);
+  {
+    const rawl* msrc = static_cast<const rawl*>(a.mem) + (b * a.segments + te.x) * dv * dk;
+    const __amdgpu_buffer_rsrc_t rm = make_rsrc(msrc, static_cast<uint32_t>(dv * dk * sizeof(rawl)));
+    constexpr int EPU = 16 / static_cast<int>(sizeof(rawl));
+    constexpr int UNITS = (FRAGS + AL_WAVES - 1) / AL_WAVES;  // fragments per wave
+    float x[UNITS][8];
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int f = w + AL_WAVES * u, c = f % NSTEP, i = f / NSTEP;
+      const int v = v0 + 32 * (i >> 1) + 8 * (n >> 2) + 4 * (i & 1) + (n & 3), k = 32 * c + 8 * g;
+#pragma unroll
+      for (int h = 0; h < 8; h += EPU)
+        load16_f32<EL>(rm, (i < NI && v < dv && k + h < dk) ? (v * dk + k + h) * static_cast<int>(sizeof(rawl)) : kBufOOB,
+                       &x[u][h]);
+    }
+#pragma unroll
+    for (int u = 0; u < UNITS; ++u) {
+      const int f = w + AL_WAVES * u, c = f % NSTEP, i = f / NSTEP;
+      if (i >= NI) continue;
+#pragma unroll
+      for (int part = 0; part < NPART; ++part) {
+        Frag8<EF> fr;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const rawf h = ET<EF>::from_f(x[u][e]);
+          fr.e[e] = h;
+          x[u][e] -= ET<EF>::to_f(h);
+        }
+        As[((part * NSTEP + c) * NI + i) * 64 + lane] = fr;
+      }
+    }
+  }
+
+  const __amdgpu_buffer_rsrc_t rq =
+      make_rsrc(static_cast<const rawf*>(a.queries) + b * a.n_query * dk, static_cast<uint32_t>(a.n_query * dk * 2));
+  Frag8<EF> bq[AL_NJ][NSTEP];
+  int qoff[AL_NJ];  // byte offsets of this lane's part of its four pairs' queries
+  auto set_q = [&](int qrow_src) {
+#pragma unroll
+    for (int j = 0; j < AL_NJ; ++j) {
+      const int qrow = __shfl(qrow_src, 16 * j + n, 64);
+      qoff[j] = qrow >= 0 ? (qrow * dk + 8 * g) * 2 : kBufOOB;
+    }
+  };
+  auto load_q = [&](int c) {
+#pragma unroll
+    for (int j = 0; j < AL_NJ; ++j)
+      bq[j][c] = __builtin_bit_cast(Frag8<EF>, __builtin_amdgcn_raw_buffer_load_b128(
+                                                   rq, 32 * c + 8 * g < dk ? qoff[j] : kBufOOB, 64 * c, 0));
+  };
+  set_q(query_of(a, pid));
+#pragma unroll
+  for (int c = 0; c < NSTEP; ++c) load_q(c);
+  __syncthreads();  // the state's fragments
+
+  while (p0 < p_end) {
+    const int pn = p0 + AL_PAIRS * AL_WAVES;
+    const int pid_after = load_id(pn + AL_PAIRS * AL_WAVES);
+    set_q(query_of(a, pid_next));
+    f32x4 acc[NI][AL_NJ];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < AL_NJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // Fragments in the order of use, AHEAD of them read before their MFMAs; the
+    // scheduling barriers keep the compiler from reading all of them first (and
+    // spilling).
+    constexpr int NF = FRAGS * NPART, AHEAD = 2;
+    Frag8<EF> am[AHEAD];
+    auto frag = [&](int f) {  // f = (c NPART + part) NI + i
+      const int c = f / (NPART * NI), part = f / NI % NPART, i = f % NI;
+      return As[((part * NSTEP + c) * NI + i) * 64 + lane];
+    };
+#pragma unroll
+    for (int f = 0; f < AHEAD; ++f) am[f] = frag(f);
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const int c = f / (NPART * NI), i = f % NI;
+      const Frag8<EF> af = am[f % AHEAD];
+      if (f + AHEAD < NF) am[f % AHEAD] = frag(f + AHEAD);
+#pragma unroll
+      for (int j = 0; j < AL_NJ; ++j) acc[i][j] = mfma8(af, bq[j][c], acc[i][j]);
+      // the next 64 pairs' keys of this step, in flight from here on
+      if ((f + 1) % (NPART * NI) == 0) load_q(c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < AL_NJ; ++j) {
+      const int pj = __shfl(pid, 16 * j + n, 64);
+      float m = 0.f;
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(acc[i][j][r]));
+      {  // over the four lanes of the pair
+        const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+        m = fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
+        const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+        m = fmaxf(__uint_as_float(s16[0]), __uint_as_float(s16[1]));
+      }
+      int ex = 0;
+      (void)frexpf(m, &ex);
+      const int sh = min(max(15 - ex, -100), 100);
+      const int ro = pj * (2 * dv) + 2 * (v0 + 8 * g);  // pj = -1: below zero, out of range
+#pragma unroll
+      for (int p = 0; p < NI / 2; ++p) {
+        u32x4 q;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 y = acc[2 * p + h][j];
+          q[2 * h] = pack2<F16>(ldexpf(y[0], sh), ldexpf(y[1], sh));
+          q[2 * h + 1] = pack2<F16>(ldexpf(y[2], sh), ldexpf(y[3], sh));
+        }
+        // (the offset in the vector register: with 64 p as the scalar offset the compiler
+        // counts no wait state between the store and the next write to q, and now and
+        // then a row's first dword of 16 bytes was the next piece's)
+        __builtin_amdgcn_raw_buffer_store_b128(q, rout, v0 + 32 * p + 8 * g < dv ? ro + 64 * p : kBufOOB, 0, 0);
+      }
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ldexpf(1.f, -sh)), rscale,
+                                            g == 0 ? (pj * a.v_tiles + static_cast<int>(vt)) * 4 : kBufOOB, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    p0 = pn;
+    pid = pid_next;
+    pid_next = pid_after;
+  }
+}
+
+template <class EL, class EQ, int DKP, class EF, int NPART, int NI>
+int launch_apply_lds(const RetrieveArgs& a, hipStream_t s) {
+  constexpr size_t lds = static_cast<size_t>(NPART) * (DKP / 32) * NI * 64 * 16;
+  static_assert(lds <= 160 * 1024, "the state's parts fit one CU's LDS");
+  if (lds > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(&apply_lds_kernel<EL, EQ, DKP, EF, NPART, NI>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    if (e != hipSuccess) {
+      set_error("retrieve_fuse: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+      return static_cast<int>(e);
+    }
+  }
+  const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(a.tb_max) * a.v_tiles), static_cast<unsigned>(a.batch));
+  hipLaunchKernelGGL((apply_lds_kernel<EL, EQ, DKP, EF, NPART, NI>), grid, dim3(AL_THREADS), lds, s, a);
+  return check_launch("retrieve_fuse(apply)");
+}
+
+// The state in LDS wherever several workgroups share a CU (up to 48 KB of parts:
+// 4 x 4000 queries, 8 of 63 states of 512 x 64, 147 -> 121 us; 8 x 2000, 8 of 200 of
+// 64 x 64, 57 -> 47 us).  Larger states leave one or two workgroups per CU, whose
+// staging nothing hides: from 256 pairs per state on (128 x 128 float32 states, 64
+// pairs 460 -> 606 us, 128 pairs 222 -> 239, 256 pairs 351 -> 347, 512 pairs 604 -> 555).
+// The buffer offsets of that kernel are 32 bits.
+template <class EL, class EQ, int DKP, class EF, int NPART, int NI>
+int launch_scaled_rows(const RetrieveArgs& a, hipStream_t s) {
+  constexpr bool kShared = NPART * (DKP / 32) * NI <= 48;  // fragments of 1 KB
+  if ((kShared || a.mean_pairs >= kLdsApplyPairs) && a.n_index * a.dv * 2 <= INT32_MAX &&
+      static_cast<int64_t>(a.tb_max) * a.v_tiles * AL_THREADS <= UINT32_MAX)
+    return launch_apply_lds<EL, EQ, DKP, EF, NPART, NI>(a, s);
+  return launch_apply_mfma16<EL, F32, EQ, DKP, EF, NPART, true>(a, s);
+}
+
+template <class EL, class EQ, int DKP, class EF, int NPART>
+int launch_scaled_width(const RetrieveArgs& a, hipStream_t s) {
+  if (a.dv <= 32) return launch_scaled_rows<EL, EQ, DKP, EF, NPART, 2>(a, s);
+  if (a.dv <= 64) return launch_scaled_rows<EL, EQ, DKP, EF, NPART, 4>(a, s);
+  return launch_scaled_rows<EL, EQ, DKP, EF, NPART, 8>(a, s);
+}
+
 // The scaled apply runs the exact 16-bit MFMA kernel with float32 arithmetic;
 // other dtype pairs and unaligned shapes are not supported by retrieve_fuse.
 template <class EL, class EQ>
@@ -1010,9 +1281,9 @@ int launch_apply_scaled(const RetrieveArgs& a, hipStream_t s) {
   if constexpr (Plan::ok) {
     using EF = typename Plan::EF;
     constexpr int NPART = Plan::parts;
-    if (a.dk <= 32) return launch_apply_mfma16<EL, F32, EQ, 32, EF, NPART, true>(a, s);
-    if (a.dk <= 64) return launch_apply_mfma16<EL, F32, EQ, 64, EF, NPART, true>(a, s);
-    return launch_apply_mfma16<EL, F32, EQ, 128, EF, NPART, true>(a, s);
+    if (a.dk <= 32) return launch_scaled_width<EL, EQ, 32, EF, NPART>(a, s);
+    if (a.dk <= 64) return launch_scaled_width<EL, EQ, 64, EF, NPART>(a, s);
+    return launch_scaled_width<EL, EQ, 128, EF, NPART>(a, s);
   } else {
     set_error("retrieve_fuse: no exact 16-bit MFMA plan for these dtypes");
     return GRM_HIP_EUNSUPPORTED;
@@ -1461,12 +1732,14 @@ int64_t partial_bytes(int64_t batch, int64_t segments, int64_t n_index) {
   return c > 1 ? (batch * c * segments * 4 + 15) / 16 * 16 : 0;
 }
 
-// Pairs per apply work tile: the mean pairs per segment (at least 512, a
-// multiple of the 64-pair MFMA tile), so balanced selections keep about one
-// tile per segment and a heavily selected segment is split.
+// Pairs per apply work tile: one and a half times the mean pairs per segment (at
+// least 512, a multiple of the 64-pair MFMA tile), so balanced selections keep one
+// tile per segment and a heavily selected segment is split.  At the mean itself
+// half of the segments had a second tile of a few pairs that read the state again
+// (16 x 65536 queries over 512 states: 3.97 -> 3.67 ms).
 int64_t tile_pairs_for(int64_t segments, int64_t n_index) {
   const int64_t mean = segments > 0 ? (n_index + segments - 1) / segments : n_index;
-  const int64_t tp = (mean + AP_N - 1) / AP_N * AP_N;
+  const int64_t tp = (mean + mean / 2 + AP_N - 1) / AP_N * AP_N;
   return tp > 8 * AP_N ? tp : 8 * AP_N;
 }
 
@@ -1522,6 +1795,7 @@ void init_retrieve_args(RetrieveArgs& a, const void* memories, const int64_t* in
   a.n_index = n_index;
   a.dv = static_cast<int>(hidden_size);
   a.dk = static_cast<int>(key_dim);
+  a.mean_pairs = static_cast<int>(segments > 0 ? n_index / segments : n_index);
   a.out_row = a.dv;
   a.v_tiles = static_cast<int>((hidden_size + AP_V - 1) / AP_V);
 }
@@ -1669,7 +1943,6 @@ extern "C" int grm_hip_retrieve_fuse(const void* memories, const int64_t* indice
     RetrieveArgs a;
     init_retrieve_args(a, memories, indices, queries, rows16, workspace, batch, segments, n_query, routes, n_index,
                        value_dim, key_dim, bad_index_count);
-    a.gates = gates;
     a.scales = scales;
     if (!scaled_supported(a, mem_dtype, q_dtype)) {
       set_error("retrieve_fuse: needs bf16 queries (or f16 queries with f16 memories), 16-byte rows and "
@@ -1691,6 +1964,7 @@ extern "C" int grm_hip_retrieve_fuse(const void* memories, const int64_t* indice
   f.h = h_online;
   f.rows = reinterpret_cast<const uint16_t*>(rows16);
   f.scales = scales;
+  f.gates = gates;
   f.w = ln_weight;
   f.bias = ln_bias;
   f.out = out;

@@ -583,6 +583,43 @@ def _retrieve_fuse_ref(mem, idx, q, gates, h, w, b, eps=1e-5):
                              eps).reshape(B, Q, H)
 
 
+@pytest.mark.parametrize("mem_dtype,q_dtype", [(torch.float32, torch.bfloat16), (torch.float16, torch.bfloat16),
+                                               (torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("B,Q,S,R,H,K", [(1, 1, 3, 1, 8, 32), (1, 47, 1, 1, 32, 32), (2, 49, 2, 2, 64, 40),
+                                         (1, 300, 1, 1, 128, 128), (1, 385, 1, 1, 128, 128),
+                                         (2, 1700, 2, 2, 136, 120), (1, 5000, 5, 4, 512, 64), (1, 9000, 3, 8, 72, 16)])
+def test_retrieve_fuse_states_in_lds(dev, mem_dtype, q_dtype, B, Q, S, R, H, K):
+    """retrieve_fuse where a state is kept in LDS for many pairs: fewer pairs than a wave takes,
+    one more than one and than eight waves take (48, 384), value widths of every padded size with
+    partial tiles, key widths below the padded ones, several work tiles per state, sorts over one
+    workgroup and over several (65536 pairs on); states of very different magnitude, and pairs with
+    an invalid index whose gate is NaN (absent, whatever its gate).  Rows are kept as float16 scaled
+    by their largest value: 2^-11 of it each, R of them summed under gates that add to one, before
+    a LayerNorm of unit scale, so 2e-3 of the output's largest value bounds the error."""
+    g = torch.Generator().manual_seed(Q + H)
+    mem = torch.randn(B, S, H, K, generator=g) * 0.3
+    mem[:, 0] *= 2.0 ** (-12 if mem_dtype == torch.float16 else -60)
+    mem = mem.to(mem_dtype)
+    idx = torch.stack([torch.stack([torch.randperm(S, generator=g)[:R] if R <= S else
+                                    torch.randint(0, S, (R,), generator=g) for _ in range(Q)]) for _ in range(B)])
+    q = norm(torch.randn(B, Q, K, generator=g)).to(q_dtype)
+    gates = torch.softmax(torch.randn(B, Q, R, generator=g), dim=-1)
+    h = torch.randn(B, Q, H, generator=g)
+    w, b = 1 + 0.1 * torch.randn(H, generator=g), 0.1 * torch.randn(H, generator=g)
+    if Q > 1:
+        idx[0, 1, 0], idx[-1, -1, -1] = -1, S
+    ref = _retrieve_fuse_ref(mem, idx, q, gates, h, w, b)
+    if Q > 1:
+        gates[0, 1, 0] = gates[-1, -1, -1] = float("nan")
+    print(f"retrieve_fuse states in LDS B={B} Q={Q} S={S} R={R} H={H} K={K} {mem_dtype} {q_dtype}", flush=True)
+    args = [t.to(dev) for t in (mem, idx, q, gates, h, w, b)]
+    out, again = capi.retrieve_fuse(*args), capi.retrieve_fuse(*args)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    got = out.double().cpu().numpy()
+    assert np.abs(got - ref).max() <= 2e-3 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("mem_dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("h_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,Q,S,R,H,K,ln", [(2, 300, 37, 5, 128, 128, True), (3, 64, 8, 8, 512, 64, True),
