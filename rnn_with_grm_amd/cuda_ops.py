@@ -312,6 +312,10 @@ class _SegmentScanFn(torch.autograd.Function):
         states = snapshots if int(segment_len) == _STATE_CHUNK else memory.new_empty(0)
         ctx.save_for_backward(keys, values, queries, memory, states)
         ctx.mark_non_differentiable(snapshots)
+        # Without this autograd fills a zero gradient as large as the snapshots for every
+        # backward (64 x 2048 tokens of width 128: 134 MB, 19 of 270 us); _scan_grads takes
+        # absent gradients of the other outputs as zeros.
+        ctx.set_materialize_grads(False)
         return hidden, memory_out, snapshots
 
     @staticmethod

@@ -430,6 +430,23 @@ def test_float32_backward(dev, dtype, mem_dtype, shift, B, T, K, H):
             close_elementwise(name, x, r)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_segment_scan_gradient_of_one_output(dev, dtype):
+    """cuda_segment_scan when only one of its two differentiable outputs enters the loss (the other's
+    gradient is absent, and the snapshots' is never made): the same gradients as with explicit zeros
+    for the other, bit for bit."""
+    k, v, q, m = make_case(2, 150, 32, 64, dtype, torch.float32, seed=5)
+    ins = [t.to(dev).requires_grad_(True) for t in (k, v, q, m)]
+    hidden, memory, _ = cuda_ops.cuda_segment_scan(*ins, 0.97, 64)
+    g = torch.Generator().manual_seed(6)
+    gh = torch.randn(hidden.shape, generator=g).to(dtype).to(dev)
+    gm = torch.randn(memory.shape, generator=g).to(dev)
+    for one, zeros in (((hidden,), (gh, torch.zeros_like(gm))), ((memory,), (torch.zeros_like(gh), gm))):
+        alone = torch.autograd.grad(one, ins, (gh if one[0] is hidden else gm,), retain_graph=True)
+        both = torch.autograd.grad((hidden, memory), ins, zeros, retain_graph=True)
+        assert all(torch.equal(x, y) for x, y in zip(alone, both))
+
+
 def test_autograd_through_cuda_ops(dev):
     """cuda_chunk_update under autograd matches the fallback's autograd (the
     reference's check, examples/test_grm.py:72-113)."""
