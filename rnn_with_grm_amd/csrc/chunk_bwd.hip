@@ -54,8 +54,8 @@ namespace {
 // Wave w owns query/key block w (tokens [16w, +16)) of every per-chunk product.
 constexpr int MB_DV = 32;  // value columns per tile of bwd_grad_kernel
 constexpr int MB_NT = 256;
-constexpr int AJ_V = 64;   // value rows per bwd_adjoint_kernel workgroup
-constexpr int AJ_NT = 512; // bwd_adjoint_kernel: 8 waves, wave w owns value rows 16 (w & 3) .. + 16 and key half w >> 2
+constexpr int AJ_V = 64;   // value rows per bwd_adjoint_kernel workgroup (or half), and per join / fix-up workgroup
+constexpr int AJ_NT = 512; // bwd_adjoint_kernel: 8 waves, wave w owns value block w % VB and key share w / VB
 
 struct BwdMArgs {
   const void* dh;
@@ -84,17 +84,20 @@ struct BwdMArgs {
   float pw[BCT + 1];  // decay^0 .. decay^64
 };
 
-template <int DKP>
+// VB 16-row value blocks per workgroup (4, or 2: twice the workgroups, each wave
+// with a quarter of the key columns instead of a half).
+template <int DKP, int VB>
 struct AjShape {
-  static constexpr int KS = DKP + 8;   // Q rows (4 banks mod 64)
-  static constexpr int HS = AJ_V + 8;  // dH rows of the tile
+  static constexpr int V = 16 * VB;     // value rows per workgroup
+  static constexpr int KS = DKP + 8;    // Q rows (4 banks mod 64)
+  static constexpr int HS = V + 8;      // dH rows of the tile
   static constexpr int KT = DKP / 16;
   static constexpr int KU = DKP / 8;
-  static constexpr int KTW = KT / 2;   // key tiles of one wave
+  static constexpr int KTW = KT * VB / 8;  // key tiles of one wave
   static constexpr int K_UNITS = BCT * KU / AJ_NT;
-  static constexpr int H_UNITS = BCT * (AJ_V / 8) / AJ_NT;
+  static constexpr int HU = V / 8;      // 16-byte units per dH row; the first BCT HU threads stage them
   static constexpr size_t lds_bytes = static_cast<size_t>(BCT * KS + BCT * HS) * 2 + (BCT + 1) * 4;
-  static_assert(K_UNITS * AJ_NT == BCT * KU && H_UNITS * AJ_NT == BCT * (AJ_V / 8), "tiles split evenly");
+  static_assert(K_UNITS * AJ_NT == BCT * KU && BCT * HU <= AJ_NT, "tiles split evenly");
 };
 
 template <int DKP>
@@ -147,9 +150,9 @@ __device__ __forceinline__ void store4_split(typename ET<E>::raw* hi, typename E
 // The adjoint recurrence.  Lane (g, n) of wave w holds gacc[t][r] =
 // G[v][k], v = v0 + 16 w + n, k = 16 t + 4 g + r.  Chunk staging: the loads of
 // chunk ch - 1 are in flight while chunk ch is processed.
-template <class E, int DKP>
+template <class E, int DKP, int VB>
 __global__ __launch_bounds__(AJ_NT) void bwd_adjoint_kernel(const BwdMArgs a) {
-  using S = AjShape<DKP>;
+  using S = AjShape<DKP, VB>;
   using raw = typename ET<E>::raw;
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -166,7 +169,7 @@ __global__ __launch_bounds__(AJ_NT) void bwd_adjoint_kernel(const BwdMArgs a) {
   const int g = lane >> 4;
   const int n = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int vtiles = (a.dv + AJ_V - 1) / AJ_V;
+  const int vtiles = (a.dv + S::V - 1) / S::V;
   int wg = blockIdx.x;
   if (a.xcd_remap) {  // the value tiles of one sequence (same queries) on one XCD
     const int per = gridDim.x >> 3;
@@ -177,14 +180,14 @@ __global__ __launch_bounds__(AJ_NT) void bwd_adjoint_kernel(const BwdMArgs a) {
   const int64_t b = wg / vtiles / a.n_parts;
   const int c0 = part * a.cpp, c1 = min(a.n_chunks, c0 + a.cpp);  // chunks [c0, c1)
   const bool last_part = part == a.n_parts - 1;
-  const int v0 = tile * AJ_V;
+  const int v0 = tile * S::V;
   const int dk = a.dk, dv = a.dv;
   const int64_t T = a.T;
   const int last_len = static_cast<int>(T - static_cast<int64_t>(a.n_chunks - 1) * BCT);
   const raw* queries = static_cast<const raw*>(a.queries) + b * T * dk;
   const raw* dh = static_cast<const raw*>(a.dh) + b * T * dv;
   if (tid <= BCT) pw[tid] = a.pw[tid];
-  const int wr = w & 3, kt0 = KT * (w >> 2);  // value block, first key tile of this wave
+  const int wr = w % VB, kt0 = KT * (w / VB);  // value block, first key tile of this wave
   const int vrow = v0 + 16 * wr + n;
   const int64_t mem_b = a.mem_f32 ? 4 : ES;
   auto g_off = [&](int t) -> int {
@@ -224,7 +227,7 @@ __global__ __launch_bounds__(AJ_NT) void bwd_adjoint_kernel(const BwdMArgs a) {
 
   struct Stage {
     U8<E> q[S::K_UNITS];
-    U8<E> h[S::H_UNITS];
+    U8<E> h;
   };
   auto load_chunk = [&](int ch, Stage& sg) {
     const int64_t t0 = static_cast<int64_t>(ch) * BCT;
@@ -237,12 +240,9 @@ __global__ __launch_bounds__(AJ_NT) void bwd_adjoint_kernel(const BwdMArgs a) {
       const int row = l / KU, col = 8 * (l % KU);
       sg.q[u] = buf_load8<E>(rq, col < dk ? (row * dk + col) * ES : kBufOOB);
     }
-#pragma unroll
-    for (int u = 0; u < S::H_UNITS; ++u) {
-      const int l = tid + AJ_NT * u;
-      const int row = l / (AJ_V / 8), col = 8 * (l % (AJ_V / 8));
-      sg.h[u] = buf_load8<E>(rh, v0 + col < dv ? (row * dv + v0 + col) * ES : kBufOOB);
-    }
+    // (threads past the dH tile read out of range: zeros, not stored)
+    const int row = tid / S::HU, col = 8 * (tid % S::HU);
+    sg.h = buf_load8<E>(rh, row < BCT && v0 + col < dv ? (row * dv + v0 + col) * ES : kBufOOB);
   };
   auto store_chunk = [&](const Stage& sg) {
 #pragma unroll
@@ -250,11 +250,8 @@ __global__ __launch_bounds__(AJ_NT) void bwd_adjoint_kernel(const BwdMArgs a) {
       const int l = tid + AJ_NT * u;
       *reinterpret_cast<U8<E>*>(Qs + (l / KU) * KS + 8 * (l % KU)) = sg.q[u];
     }
-#pragma unroll
-    for (int u = 0; u < S::H_UNITS; ++u) {
-      const int l = tid + AJ_NT * u;
-      *reinterpret_cast<U8<E>*>(Hs + (l / (AJ_V / 8)) * HS + 8 * (l % (AJ_V / 8))) = sg.h[u];
-    }
+    if (BCT * S::HU == AJ_NT || tid < BCT * S::HU)
+      *reinterpret_cast<U8<E>*>(Hs + (tid / S::HU) * HS + 8 * (tid % S::HU)) = sg.h;
   };
 
   // (Loading two chunks ahead, in two register stages, measured slower: 84
@@ -720,14 +717,23 @@ int allow_lds(K* fn, size_t bytes, bool& done) {
 
 template <class E, int DKP>
 int launch_bwd_mfma(BwdMArgs a, int mem_dtype, hipStream_t s) {
-  static bool attr_a = false, attr_g = false;
-  int rc = allow_lds(&bwd_adjoint_kernel<E, DKP>, AjShape<DKP>::lds_bytes, attr_a);
-  if (rc == GRM_HIP_OK) rc = allow_lds(&bwd_grad_kernel<E, DKP>, GrShape<DKP>::lds_bytes, attr_g);
+  static bool attr_g = false;
+  static_assert(AjShape<DKP, 4>::lds_bytes <= 64 * 1024, "no attribute needed");
+  int rc = allow_lds(&bwd_grad_kernel<E, DKP>, GrShape<DKP>::lds_bytes, attr_g);
   if (rc != GRM_HIP_OK) return rc;
-  const int64_t grid_a = a.batch * ((a.dv + AJ_V - 1) / AJ_V) * a.n_parts;
+  // 32-row workgroups where 64-row ones would leave CUs idle: each walks the same
+  // chunks with half the work per step (64 x 2048 tokens of width 128, 128 -> 256
+  // workgroups, 68 -> 61 us).
+  const bool narrow = a.batch * ((a.dv + AJ_V - 1) / AJ_V) * a.n_parts < 192;
+  const int rows = narrow ? AJ_V / 2 : AJ_V;
+  const int64_t grid_a = a.batch * ((a.dv + rows - 1) / rows) * a.n_parts;
   a.xcd_remap = (grid_a % 8 == 0) ? 1 : 0;
-  hipLaunchKernelGGL((bwd_adjoint_kernel<E, DKP>), dim3(static_cast<unsigned>(grid_a)), dim3(AJ_NT),
-                     AjShape<DKP>::lds_bytes, s, a);
+  if (narrow)
+    hipLaunchKernelGGL((bwd_adjoint_kernel<E, DKP, 2>), dim3(static_cast<unsigned>(grid_a)), dim3(AJ_NT),
+                       (AjShape<DKP, 2>::lds_bytes), s, a);
+  else
+    hipLaunchKernelGGL((bwd_adjoint_kernel<E, DKP, 4>), dim3(static_cast<unsigned>(grid_a)), dim3(AJ_NT),
+                       (AjShape<DKP, 4>::lds_bytes), s, a);
   rc = check_launch("chunk_update_bwd(adjoint)");
   if (rc != GRM_HIP_OK) return rc;
   if (a.n_parts > 1) {
