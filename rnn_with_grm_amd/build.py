@@ -28,9 +28,9 @@ LIB_HIP = PKG_DIR / "libgrm_hip.so"
 LIB_EXT = PKG_DIR / "grm_cuda_ext.so"
 
 OFFLOAD_ARCH = "gfx950"
-HIP_SOURCES = ["grm_capi.hip", "chunk_scan.hip", "chunk_scan_wide.hip", "chunk_scan_vsplit.hip", "chunk_bwd.hip",
-               "chunk_bwd_f32.hip", "gather_apply.hip", "retrieve.hip", "retrieve_window.hip", "route_fuse.hip",
-               "route_select.hip", "layer_glue.hip"]
+HIP_SOURCES = ["grm_capi.hip", "chunk_scan.hip", "chunk_scan_wide.hip", "chunk_scan_vsplit.hip", "chunk_scan_par.hip",
+               "chunk_bwd.hip", "chunk_bwd_f32.hip", "gather_apply.hip", "retrieve.hip", "retrieve_window.hip",
+               "route_fuse.hip", "route_select.hip", "layer_glue.hip"]
 EXT_SOURCE = "grm_torch_ops.cpp"
 
 # Packed fp32 instructions are kept out of every kernel (the flag is for the
@@ -75,8 +75,7 @@ def _stale(target: Path, deps: List[Path]) -> bool:
 
 def _headers() -> List[Path]:
     return [INCLUDE / "grm_hip.h", CSRC / "grm_hip_common.h", CSRC / "chunk_scan.h", CSRC / "chunk_bwd.h",
-            CSRC / "route_select.h",
-            CSRC / "retrieve.h"]
+            CSRC / "f32_tiles.h", CSRC / "route_select.h", CSRC / "retrieve.h"]
 
 
 def build_hip_library(force: bool = True, verbose: bool = False, jobs: Optional[int] = None) -> Path:

@@ -35,6 +35,7 @@
 #include <algorithm>
 
 #include "chunk_bwd.h"
+#include "f32_tiles.h"
 #include "grm_hip.h"
 #include "grm_hip_common.h"
 
@@ -45,64 +46,6 @@ constexpr int GNT = 256;          // threads per workgroup
 constexpr int GVS = kGenDv + 4;   // LDS row stride of the V and dH tiles
 constexpr int GPS = BCT + 4;      // LDS row stride of P and dS
 constexpr int OUTER_V = 64;       // value rows per bwd_outer_kernel workgroup
-
-__device__ __forceinline__ f32x4 mfma4(f32x4 a, f32x4 b, f32x4 acc) {
-#pragma unroll
-  for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc, 0, 0, 0);
-  return acc;
-}
-
-// Four consecutive elements of an LDS row (reduction slots 4g + s of a 16-deep step).
-template <class E>
-__device__ __forceinline__ f32x4 lds_row4(const typename ET<E>::raw* p) {
-  f32x4 r;
-  if constexpr (sizeof(typename ET<E>::raw) == 2) {
-    const uint2 u = *reinterpret_cast<const uint2*>(p);
-    r[0] = ET<E>::to_f(static_cast<uint16_t>(u.x & 0xffffu));
-    r[1] = ET<E>::to_f(static_cast<uint16_t>(u.x >> 16));
-    r[2] = ET<E>::to_f(static_cast<uint16_t>(u.y & 0xffffu));
-    r[3] = ET<E>::to_f(static_cast<uint16_t>(u.y >> 16));
-  } else {
-    const float4 u = *reinterpret_cast<const float4*>(p);
-    r[0] = u.x; r[1] = u.y; r[2] = u.z; r[3] = u.w;
-  }
-  return r;
-}
-
-// Four elements of an LDS column, rows p, p + stride, ...
-template <class E>
-__device__ __forceinline__ f32x4 lds_col4(const typename ET<E>::raw* p, int stride) {
-  f32x4 r;
-#pragma unroll
-  for (int s = 0; s < 4; ++s) r[s] = ET<E>::to_f(p[s * stride]);
-  return r;
-}
-
-// Four consecutive output elements at element `el` (`left` of them inside the row).
-template <class E>
-__device__ __forceinline__ void out4(__amdgpu_buffer_rsrc_t r, int el, int left, bool vec, f32x4 v) {
-  constexpr int ES = static_cast<int>(sizeof(typename ET<E>::raw));
-  if (vec) {
-    buf_store4<E>(r, left > 0 ? el * ES : kBufOOB, v);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) buf_store1<E>(r, i < left ? (el + i) * ES : kBufOOB, v[i]);
-  }
-}
-
-__device__ __forceinline__ float ld_mem(__amdgpu_buffer_rsrc_t r, int el, bool f32, bool ok, F32) {
-  (void)f32;
-  return buf_load1<F32>(r, ok ? el * 4 : kBufOOB);
-}
-template <class E>
-__device__ __forceinline__ float ld_mem(__amdgpu_buffer_rsrc_t r, int el, bool f32, bool ok, E) {
-  return f32 ? buf_load1<F32>(r, ok ? el * 4 : kBufOOB) : ET<E>::to_f(buf_load1<E>(r, ok ? el * 2 : kBufOOB));
-}
-
-template <class E>
-__device__ __forceinline__ float ld_state(const void* p, int64_t i, bool f32) {
-  return f32 ? static_cast<const float*>(p)[i] : ET<E>::to_f(static_cast<const typename ET<E>::raw*>(p)[i]);
-}
 
 // dH^T diag(decay^{i+1}) Q of one chunk: workgroup (sequence, chunk, 64 value
 // rows), wave w rows [16w, +16), every key column.  Operands straight from
