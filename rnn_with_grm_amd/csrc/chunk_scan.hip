@@ -637,7 +637,8 @@ struct Plan {
 // (sequence, value tile) workgroups; with more, the walk fills the chip by itself
 // without the slots' traffic.  The slots' three launches are worth about four chunks of
 // the walk at key_dim 64 (32 x 256 tokens, value_dim 128: 22.0 us walked, 22.6 over slots;
-// 4 x 512, 256: 35 and 22) and two at key_dim 128 (8 x 256, 256: 35 and 23).  The slots stay within the fixed scratch of the
+// 4 x 512, 256: 35 and 22), two at key_dim 128 (8 x 256, 256: 35 and 23) and five up to
+// 32 (4 x 320, 256: 18.9 and 20.0; 4 x 384: 21.2 and 20.1).  The slots stay within the fixed scratch of the
 // no-alloc entry point, so that both entry points take the same way.  The choice does
 // not depend on whether snapshots or a workspace are given (a call that has neither
 // room walks).  GRM_HIP_CHUNK_DV and GRM_HIP_CHUNK_PARTS ask for the walk.
@@ -647,8 +648,8 @@ Par par_plan(const Plan& p, int64_t batch, int64_t value_dim, int64_t key_dim) {
   if (p.wide || p.vsplit || getenv("GRM_HIP_CHUNK_DV") != nullptr || getenv("GRM_HIP_CHUNK_PARTS") != nullptr ||
       !par_fits(batch, p.n_chunks, value_dim, key_dim) || p.n_chunks < 1)
     return Par::kNone;
-  if (par_direct(batch, p.n_chunks, value_dim)) return Par::kDirect;
-  if (batch * p.v_tiles < 192 && p.n_chunks > (key_dim > 64 ? 2 : 4) &&
+  if (par_direct(batch, p.n_chunks, value_dim, key_dim)) return Par::kDirect;
+  if (batch * p.v_tiles < 192 && p.n_chunks > (key_dim > 64 ? 2 : key_dim > 32 ? 4 : 5) &&
       par_slot_bytes(batch, p.n_chunks, value_dim, key_dim) <= GRM_HIP_NOALLOC_SCRATCH_BYTES)
     return Par::kSlots;
   return Par::kNone;

@@ -5,7 +5,7 @@
 // Walking a sequence chunk by chunk costs 4-5 us per 64-token chunk (a chain of LDS
 // round trips and float32 MFMAs), and the S = Q K^T of a chunk is repeated for every
 // 32-column value tile.  Here a workgroup takes one chunk:
-//   up to kParDirectChunks chunks: one launch (fwd_chunk_kernel<.., true>).  Each
+//   few chunks (par_direct): one launch (fwd_chunk_kernel<.., true>).  Each
 //     workgroup forms the state at its chunk's start itself, by walking the earlier
 //     chunks' K and V (no S, no outputs), then its outputs; one more per sequence
 //     forms the last state.
@@ -474,8 +474,11 @@ int64_t par_slot_bytes(int64_t batch, int64_t n_chunks, int64_t value_dim, int64
   return batch * n_chunks * value_dim * key_dim * 4;
 }
 
-bool par_direct(int64_t batch, int64_t n_chunks, int64_t value_dim) {
-  return n_chunks <= kParDirectChunks && batch * (n_chunks + 1) * ((value_dim + PDV - 1) / PDV) <= kParDirectWgs;
+// Up to six chunks, eight of narrow keys, and one workgroup per CU: 4 x 256 tokens (64, 256)
+// 15.1 us against 21.1 over slots and 20.6 walked, 4 x 384 (64, 128) 19.1 / 19.3 / 27.4, 4 x 448
+// (32, 256) 17.6 / 20.1 / 23.6; eight chunks of 64 keys 26.5 / 22.4 / 35.
+bool par_direct(int64_t batch, int64_t n_chunks, int64_t value_dim, int64_t key_dim) {
+  return n_chunks <= (key_dim > 32 ? 6 : 8) && batch * (n_chunks + 1) * ((value_dim + PDV - 1) / PDV) <= kParDirectWgs;
 }
 
 bool par_fits(int64_t batch, int64_t n_chunks, int64_t value_dim, int64_t key_dim) {

@@ -289,11 +289,12 @@ def test_long_context_split_fp32(dev, monkeypatch):
 @pytest.mark.parametrize("dtype,mem_dtype,shift", [(torch.float32, torch.float32, 0), (torch.float32, torch.float32, 1),
                                                    (torch.bfloat16, torch.float32, 1), (torch.float16, torch.float16, 1)])
 @pytest.mark.parametrize("B,T,K,H,seg", [(1, 1, 8, 16, 0), (2, 64, 25, 31, 64), (2, 65, 32, 33, 64), (3, 500, 33, 100, 100),
-                                         (1, 256, 64, 257, 128), (2, 257, 65, 64, 64), (4, 1300, 128, 40, 0),
+                                         (1, 384, 64, 257, 128), (2, 385, 65, 64, 64),
+                                         (2, 512, 32, 40, 64), (2, 513, 20, 36, 0), (4, 1300, 128, 40, 0),
                                          (1, 2000, 64, 96, 64), (3, 700, 16, 64, 50), (1, 640, 128, 20, 1000)])
 def test_chunk_parallel_scan(dev, dtype, mem_dtype, shift, B, T, K, H, seg):
     """The chunk-parallel scan against the oracle: one token, one full chunk, ragged last chunks,
-    up to four chunks (one launch) and more (state slots, in the snapshots or in the workspace),
+    few chunks (one launch: up to six, eight of narrow keys) and more (state slots, in the snapshots or in the workspace),
     key widths on both sides of each padded width, value widths that are no multiple of the
     32-column tile, snapshots every chunk, every other one, at shorter chunks and once, rows that
     start one element past an aligned address (shift); and the same bits with and without snapshots
