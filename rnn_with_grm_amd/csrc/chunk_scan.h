@@ -103,13 +103,10 @@ bool vsplit_supported(int in_dtype, int64_t key_dim, int64_t value_dim, bool vec
 // Launches the value-split kernel (a.n_parts must be 1, a.v_tiles = value_dim / kVsplitDv).
 int launch_scan_vsplit(const ChunkFwdArgs& a, int in_dtype, hipStream_t stream);
 
-// The chunk-parallel scan (chunk_scan_par.hip).  With few chunks in few workgroups it is
-// one launch with slots == nullptr (par_direct); else it keeps the state
-// after every chunk in slots (par_slot_bytes: the caller's snapshots when one follows every
-// chunk, or workspace).  vec_k / vec_v: rows of dk / dv elements allow 4-element stores.
-int64_t par_slot_bytes(int64_t batch, int64_t n_chunks, int64_t value_dim, int64_t key_dim);
+// The chunk-parallel scan (chunk_scan_par.hip): float32 inputs with few chunks in few
+// workgroups (par_direct), one launch, the walk's results bit for bit.  vec_k / vec_v: rows
+// of dk / dv elements allow 4-element stores.
 bool par_direct(int64_t batch, int64_t n_chunks, int64_t value_dim, int64_t key_dim);
-bool par_fits(int64_t batch, int64_t n_chunks, int64_t value_dim, int64_t key_dim);
-int launch_scan_par(const ChunkFwdArgs& f, int in_dtype, float* slots, bool vec_k, bool vec_v, hipStream_t s);
+int launch_scan_par(const ChunkFwdArgs& f, int in_dtype, bool vec_k, bool vec_v, hipStream_t s);
 
 }  // namespace grmhip

@@ -25,7 +25,6 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -632,29 +631,6 @@ struct Plan {
   int64_t workspace_bytes;
 };
 
-// How the chunk-parallel scan takes the work of the 16/32-column kernel: not at all,
-// in one launch, or over state slots.  It does where that kernel has fewer than 192
-// (sequence, value tile) workgroups; with more, the walk fills the chip by itself
-// without the slots' traffic.  The slots' three launches are worth about four chunks of
-// the walk at key_dim 64 (32 x 256 tokens, value_dim 128: 22.0 us walked, 22.6 over slots;
-// 4 x 512, 256: 35 and 22), two at key_dim 128 (8 x 256, 256: 35 and 23) and five up to
-// 32 (4 x 320, 256: 18.9 and 20.0; 4 x 384: 21.2 and 20.1).  The slots stay within the fixed scratch of the
-// no-alloc entry point, so that both entry points take the same way.  The choice does
-// not depend on whether snapshots or a workspace are given (a call that has neither
-// room walks).  GRM_HIP_CHUNK_DV and GRM_HIP_CHUNK_PARTS ask for the walk.
-enum class Par { kNone, kDirect, kSlots };
-
-Par par_plan(const Plan& p, int64_t batch, int64_t value_dim, int64_t key_dim) {
-  if (p.wide || p.vsplit || getenv("GRM_HIP_CHUNK_DV") != nullptr || getenv("GRM_HIP_CHUNK_PARTS") != nullptr ||
-      !par_fits(batch, p.n_chunks, value_dim, key_dim) || p.n_chunks < 1)
-    return Par::kNone;
-  if (par_direct(batch, p.n_chunks, value_dim, key_dim)) return Par::kDirect;
-  if (batch * p.v_tiles < 192 && p.n_chunks > (key_dim > 64 ? 2 : key_dim > 32 ? 4 : 5) &&
-      par_slot_bytes(batch, p.n_chunks, value_dim, key_dim) <= GRM_HIP_NOALLOC_SCRATCH_BYTES)
-    return Par::kSlots;
-  return Par::kNone;
-}
-
 // The wide kernel unless GRM_HIP_CHUNK_DV asks for the 16/32-column tiles.
 bool use_wide(int in_dtype, int64_t key_dim, int64_t value_dim, bool vec) {
   const char* env = getenv("GRM_HIP_CHUNK_DV");
@@ -703,10 +679,7 @@ extern "C" int64_t grm_hip_chunk_update_fwd_workspace(int64_t batch, int64_t seq
   const Plan narrow = make_plan(batch, seq_len, value_dim, key_dim, snapshot_len, vec, false);
   const Plan wide = make_plan(batch, seq_len, value_dim, key_dim, snapshot_len, vec,
                               use_wide(GRM_HIP_BF16, key_dim, value_dim, vec));
-  int64_t bytes = narrow.workspace_bytes > wide.workspace_bytes ? narrow.workspace_bytes : wide.workspace_bytes;
-  if (snapshot_len != narrow.chunk && par_plan(narrow, batch, value_dim, key_dim) == Par::kSlots)
-    bytes = std::max(bytes, par_slot_bytes(batch, narrow.n_chunks, value_dim, key_dim));
-  return bytes;
+  return narrow.workspace_bytes > wide.workspace_bytes ? narrow.workspace_bytes : wide.workspace_bytes;
 }
 
 extern "C" int grm_hip_chunk_update_fwd(const void* keys, const void* values, const void* queries,
@@ -780,13 +753,9 @@ extern "C" int grm_hip_chunk_update_fwd(const void* keys, const void* values, co
     set_error("chunk_update_fwd: seq_len too large");
     return GRM_HIP_EINVAL;
   }
-  const Par par = par_plan(plan, batch, value_dim, key_dim);
-  float* slots = nullptr;
-  if (par == Par::kSlots) {
-    const int64_t need = par_slot_bytes(batch, plan.n_chunks, value_dim, key_dim);
-    if (snapshots != nullptr && snapshot_len == plan.chunk) slots = snapshots;
-    else if (workspace != nullptr && workspace_bytes >= need && aligned(workspace, 16)) slots = static_cast<float*>(workspace);
-  }
+  // GRM_HIP_CHUNK_DV and GRM_HIP_CHUNK_PARTS ask for the walk.
+  const bool par = in_dtype == GRM_HIP_F32 && getenv("GRM_HIP_CHUNK_DV") == nullptr &&
+                   getenv("GRM_HIP_CHUNK_PARTS") == nullptr && par_direct(batch, plan.n_chunks, value_dim, key_dim);
   // Without room for the per-part states, one workgroup walks each whole sequence.
   if (plan.n_parts > 1 && (workspace == nullptr || workspace_bytes < plan.workspace_bytes ||
                            !aligned(workspace, 16))) {
@@ -831,9 +800,9 @@ extern "C" int grm_hip_chunk_update_fwd(const void* keys, const void* values, co
     }
     return GRM_HIP_OK;
   }
-  if (par == Par::kDirect || slots != nullptr) {
-    const bool vk = key_dim % 4 == 0 && aligned(memory_out, 16) && aligned(snapshots, 16) && aligned(slots, 16);
-    return launch_scan_par(a, in_dtype, slots, vk, value_dim % 4 == 0 && aligned(hidden, 16), s);
+  if (par) {
+    const bool vk = key_dim % 4 == 0 && aligned(memory_out, 16) && aligned(snapshots, 16);
+    return launch_scan_par(a, in_dtype, vk, value_dim % 4 == 0 && aligned(hidden, 16), s);
   }
   if (plan.vsplit) return launch_scan_vsplit(a, in_dtype, s);
   if (plan.wide) return launch_scan_wide(a, in_dtype, mem_dtype, s);
