@@ -1048,9 +1048,9 @@ namespace {
 // Many pairs per state, for the scaled rows of retrieve_fuse: the state's MFMA
 // operands in LDS, the pairs in registers.  Eight waves stage one 16 NI-row value
 // tile of the segment's state as NPART exact 16-bit parts in fragment order (1 KB
-// per fragment, read back without bank conflicts), then each wave takes 64 pairs
-// at a time on its own, with no barrier: an A fragment read from LDS serves four
-// MFMAs, and a lane ends with all values of four pairs (a quarter of each row), so
+// per fragment, read back without bank conflicts), then each wave takes 48 pairs
+// at a time on its own, with no barrier: an A fragment read from LDS serves three
+// MFMAs, and a lane ends with a quarter of each of three pairs' rows, so
 // the gate, the row's scale and the 16-bit rows come straight from the
 // accumulators.  Row m = 4 g' + r of fragment i stands for value 32 (i >> 1) + 8 g' +
 // 4 (i & 1) + r: lane (g, n)'s accumulators of fragments 2p and 2p + 1 are then the
@@ -1102,7 +1102,7 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
     return p + lane < p_end ? id : -1;
   };
 
-  // Pair ids (one per lane) of this wave's first 64 pairs, ids of the next.
+  // Pair ids (one per lane) of this wave's first 48 pairs, ids of the next.
   int p0 = te.y + AL_PAIRS * w;
   int pid = load_id(p0), pid_next = load_id(p0 + AL_PAIRS * AL_WAVES);
   {
@@ -1141,7 +1141,7 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
   const __amdgpu_buffer_rsrc_t rq =
       make_rsrc(static_cast<const rawf*>(a.queries) + b * a.n_query * dk, static_cast<uint32_t>(a.n_query * dk * 2));
   Frag8<EF> bq[AL_NJ][NSTEP];
-  int qoff[AL_NJ];  // byte offsets of this lane's part of its four pairs' queries
+  int qoff[AL_NJ];  // byte offsets of this lane's part of its three pairs' queries
   auto set_q = [&](int qrow_src) {
 #pragma unroll
     for (int j = 0; j < AL_NJ; ++j) {
@@ -1187,7 +1187,7 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
       if (f + AHEAD < NF) am[f % AHEAD] = frag(f + AHEAD);
 #pragma unroll
       for (int j = 0; j < AL_NJ; ++j) acc[i][j] = mfma8(af, bq[j][c], acc[i][j]);
-      // the next 64 pairs' keys of this step, in flight from here on
+      // the next 48 pairs' keys of this step, in flight from here on
       if ((f + 1) % (NPART * NI) == 0) load_q(c);
       __builtin_amdgcn_sched_barrier(0);
     }
