@@ -599,6 +599,10 @@ __global__ __launch_bounds__(AP_THREADS) void apply_reg_kernel(const RetrieveArg
 // takes keys 32c + 8g .. + 7 from lane group g, so the four groups of a row
 // read consecutive bytes: each state load instruction covers whole 128-byte
 // lines of 16 rows (fp32 states) instead of 16-byte pieces of 64 lines.
+// A step of up to 32 pairs leaves out the products and stores of its upper half:
+// with about 64 pairs per state every other state ends on a step of a few (64 x 2048
+// queries, 8 of 256 states of 128 x 128: 461 -> 455 us for the whole call; tested
+// every 16 pairs, 460 us).
 template <class EL, class EM, class EQ, int DKP, class EF, int NPART, bool SCALED = false>
 __global__ __launch_bounds__(AP_THREADS) void apply_mfma16_kernel(const RetrieveArgs a) {
   using rawl = typename ET<EL>::raw;  // stored memories
@@ -686,7 +690,7 @@ __global__ __launch_bounds__(AP_THREADS) void apply_mfma16_kernel(const Retrieve
   };
   load_q(pid_l);
   for (int p0 = p_begin; p0 < p_end; p0 += AP_N) {
-    const int np = min(AP_N, p_end - p0);
+    const int np = __builtin_amdgcn_readfirstlane(min(AP_N, p_end - p0));
     const int pid_cur = pid_l;
     const bool more = p0 + AP_N < p_end;
     const int pid_next = (more && lane < p_end - p0 - AP_N) ? lb[p0 + AP_N + lane] : -1;
@@ -714,6 +718,7 @@ __global__ __launch_bounds__(AP_THREADS) void apply_mfma16_kernel(const Retrieve
       for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      if (j == 2 && np <= 32) break;  // no pairs in the upper half
       Frag8<EF> bq[NSTEP];
 #pragma unroll
       for (int c = 0; c < NSTEP; ++c) {
@@ -743,6 +748,7 @@ __global__ __launch_bounds__(AP_THREADS) void apply_mfma16_kernel(const Retrieve
     constexpr int PER = AP_N * (AP_V / 4) / AP_THREADS;  // stores per thread per full tile
 #pragma unroll
     for (int it = 0; it < PER; ++it) {
+      if (it == PER / 2 && np <= 32) break;
       const int e = tid + AP_THREADS * it;
       const int p = e / (AP_V / 4), v = (e % (AP_V / 4)) * 4;
       const int pid = __shfl(pid_cur, p, 64);

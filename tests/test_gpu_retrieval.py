@@ -583,6 +583,28 @@ def _retrieve_fuse_ref(mem, idx, q, gates, h, w, b, eps=1e-5):
                              eps).reshape(B, Q, H)
 
 
+@pytest.mark.parametrize("pairs", [1, 31, 32, 33, 63, 64, 65, 96, 97, 130])
+def test_retrieve_partial_steps(dev, pairs):
+    """States of 128 x 128 with few pairs each, whose last step of up to 64 pairs is empty, half
+    filled, one more than half and full: retrieve_fuse at the bound of test_retrieve_fuse_states_in_lds,
+    gather_apply (float32 sums of 128 exact products) at 1e-5 of its largest value."""
+    g = torch.Generator().manual_seed(pairs)
+    mem = torch.randn(1, 2, 128, 128, generator=g) * 0.3
+    idx = torch.zeros(1, pairs + 5, 1, dtype=torch.int64)
+    idx[0, pairs:] = 1
+    q = norm(torch.randn(1, pairs + 5, 128, generator=g)).to(torch.bfloat16)
+    gates, h = torch.ones(1, pairs + 5, 1), torch.randn(1, pairs + 5, 128, generator=g)
+    w, b = 1 + 0.1 * torch.randn(128, generator=g), 0.1 * torch.randn(128, generator=g)
+    print(f"retrieve partial steps {pairs}", flush=True)
+    out = capi.retrieve_fuse(*[t.to(dev) for t in (mem, idx, q, gates, h, w, b)])
+    rows = capi.gather_apply(*[t.to(dev) for t in (mem, idx, q)])
+    torch.cuda.synchronize()
+    ref = _retrieve_fuse_ref(mem, idx, q, gates, h, w, b)
+    assert np.abs(out.double().cpu().numpy() - ref).max() <= 2e-3 * np.abs(ref).max()
+    want = torch.einsum("qvk,qk->qv", mem[0, idx[0, :, 0]].double(), q[0].double()).numpy()
+    assert np.abs(rows[0, :, 0].double().cpu().numpy() - want).max() <= 1e-5 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("mem_dtype,q_dtype", [(torch.float32, torch.bfloat16), (torch.float16, torch.bfloat16),
                                                (torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16)])
 @pytest.mark.parametrize("B,Q,S,R,H,K", [(1, 1, 3, 1, 8, 32), (1, 47, 1, 1, 32, 32), (2, 49, 2, 2, 64, 40),
