@@ -37,15 +37,14 @@ struct MfmaPlan {
 };
 
 // Residual + LayerNorm over scaled float16 rows:
-//   out[t] = LN(h[t] + sum_r gates[t, r] scales[t, r, c / kScaledTile] * rows[t, r, c])
-// h and out in the h dtype, gates float32 (NULL: ones), a scale of 0 for a row that
-// is not there, the LayerNorm weight and bias float32 (w NULL: no LayerNorm), the sum
-// over r in order 0 .. R-1, a two-pass mean / variance in fp32.
+//   out[t] = LN(h[t] + sum_r scales[t, r, c / kScaledTile] * rows[t, r, c])
+// h and out in the h dtype, a scale of 0 for a row that is not there, the LayerNorm
+// weight and bias float32 (w NULL: no LayerNorm), the sum over r in order 0 .. R-1,
+// a two-pass mean / variance in fp32.
 struct FuseScaledArgs {
   const void* h;
   const uint16_t* rows;
   const float* scales;
-  const float* gates;
   const void* w;
   const void* bias;
   void* out;
@@ -53,6 +52,7 @@ struct FuseScaledArgs {
   int routes;
   int hidden;
   int v_tiles;
+  int all_there;  // no scale is 0
   float eps;
 };
 

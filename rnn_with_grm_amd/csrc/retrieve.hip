@@ -66,9 +66,11 @@ struct RetrieveArgs {
   int32_t* tile_base;
   int tb_max;
   int tile_pairs;
-  // Row-scaled 16-bit output (retrieve_fuse): out holds float16 rows of M q
-  // scaled by 2^sh per (pair, 128-value tile), scales[pair, tile] = 2^-sh, 0 for
-  // a pair without a row.  nullptr: the plain [pairs, dv] output of gather_apply.
+  // Gate-weighted, row-scaled 16-bit output (retrieve_fuse): out holds float16
+  // rows of g * M q scaled by 2^sh per (pair, 128-value tile), scales[pair, tile] =
+  // 2^-sh, 0 for a pair without a row.  nullptr: the plain [pairs, dv] output of
+  // gather_apply.
+  const float* gates;  // [batch, n_index]
   float* scales;       // [batch, n_index, v_tiles]
   int mean_pairs;  // pairs per segment, evenly spread
   int out_row;         // elements per output row (dv; dk for the queries' gradient)
@@ -215,8 +217,8 @@ __global__ __launch_bounds__(BK_THREADS) void bucket_kernel(const RetrieveArgs a
 // are read together.
 // Scaled rows: group c holds consecutive blocks of BK_THREADS pairs, so that a
 // segment's list follows the queries (in steps of a group) and workgroups on
-// different segments sweep them together (16 x 65536 queries over 512 states, with
-// the gates moved to the fusion: 3.60 -> 3.49 ms).
+// different segments sweep them together (16 x 65536 queries over 512 states, 16
+// routes each: 3.60 -> 3.49 ms).
 // Plain rows: group c holds the blocks c, c + bk_chunks, c + 2 bk_chunks, ...:
 // the empty slots of the first segments' short windows, which can fill most of
 // the first 16384 pairs, are then zeroed by every group instead of one or two.
@@ -694,6 +696,9 @@ __global__ __launch_bounds__(AP_THREADS) void apply_mfma16_kernel(const Retrieve
     const int pid_cur = pid_l;
     const bool more = p0 + AP_N < p_end;
     const int pid_next = (more && lane < p_end - p0 - AP_N) ? lb[p0 + AP_N + lane] : -1;
+    // The gate of this lane's pair, loaded while the tile's products run.
+    float gate_cur = 0.f;
+    if constexpr (SCALED) gate_cur = pid_cur >= 0 ? a.gates[b * a.n_index + pid_cur] : 0.f;
     if (!split) {
       split = true;
 #pragma unroll
@@ -754,9 +759,10 @@ __global__ __launch_bounds__(AP_THREADS) void apply_mfma16_kernel(const Retrieve
       const int pid = __shfl(pid_cur, p, 64);
       if constexpr (SCALED) {
         // The 32 lanes of one half-wave hold pair p's 128 values of this tile:
-        // scale the row so its largest magnitude lies in [2^14, 2^15) and store it
-        // as float16 with the inverse power of two.
-        const f32x4 val = *reinterpret_cast<const f32x4*>(Os + p * OS + v);
+        // scale the gate-weighted row so its largest magnitude lies in [2^14, 2^15)
+        // and store it as float16 with the inverse power of two.
+        const float gp = __shfl(gate_cur, p, 64);
+        const f32x4 val = *reinterpret_cast<const f32x4*>(Os + p * OS + v) * gp;
         float m = fmaxf(fmaxf(fabsf(val[0]), fabsf(val[1])), fmaxf(fabsf(val[2]), fabsf(val[3])));
         // maximum over the 32 lanes of the half-wave without LDS: quad swaps, the
         // half-row and row mirrors (DPP), then the 16-lane row swap
@@ -883,12 +889,10 @@ int dispatch_q(const RetrieveArgs& a, int q_dtype, hipStream_t s) {
 
 // ---------------------------------------------------------------------------
 // Residual + LayerNorm over the scaled rows of retrieve_fuse:
-//   out[t] = LN(h[t] + sum_r gates[t, r] scales[t, r, c / 128] * rows[t, r, c])
+//   out[t] = LN(h[t] + sum_r scales[t, r, c / 128] * rows[t, r, c])
 // h and out in E, the LayerNorm weight and bias in float32,
-// with r in order 0 .. R-1 (gates null: already in the rows; scale 0: no row), a
-// two-pass mean / variance in fp32.  The gates are read here, in order, rather than
-// where the rows are made, one scattered 4-byte read per pair (165 us of 2.4 ms at
-// 16 x 65536 queries with 16 routes).  lpr lanes share a row, each covering NV groups of
+// with r in order 0 .. R-1 (the gates are already in the rows; scale 0: no row), a
+// two-pass mean / variance in fp32.  lpr lanes share a row, each covering NV groups of
 // 8 consecutive columns (16-byte float16 loads of the rows).
 
 template <class E>
@@ -936,7 +940,6 @@ __global__ __launch_bounds__(256) void fuse_scaled_kernel(const FuseScaledArgs a
   const __amdgpu_buffer_rsrc_t rh = wave_rows_rsrc(a.h, wr, hb);
   const __amdgpu_buffer_rsrc_t rrow = wave_rows_rsrc(a.rows, wr, rowb);
   const float* sc = a.scales + rr * a.routes * a.v_tiles;
-  const float* ga = a.gates != nullptr ? a.gates + rr * a.routes : nullptr;
   float x[NV][8];
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
@@ -948,30 +951,28 @@ __global__ __launch_bounds__(256) void fuse_scaled_kernel(const FuseScaledArgs a
 #pragma unroll
     for (int e = 0; e < 8; ++e) r[e] = 0.f;
     const int tile = c / AP_V;
-    if (ga == nullptr && a.routes == 1) {  // the window retrieval's sums: always there
+    if (a.all_there != 0 && a.routes == 1) {  // the window retrieval's sums
       const float s0 = in ? sc[tile] : 0.f;
       float rv[8];
       load8<F16>(rrow, in ? wr.local * rowb + c * 2 : kBufOOB, rv);
 #pragma unroll
       for (int e = 0; e < 8; ++e) r[e] = fmaf(s0, rv[e], r[e]);
     } else
-    // Scale and gate of 16 routes at a time (fewer with short rows), one per lane of
+    // The scales of 16 routes at a time (fewer with short rows), one per lane of
     // the lanes on one tile; rows without a scale are not read.
     for (int j0 = 0; j0 < a.routes; j0 += per) {
       const int jl = j0 + (lane & (per - 1));
       const bool have = live && tile < a.v_tiles && jl < a.routes;  // also on lanes past the row's end
       const float sl = have ? sc[jl * a.v_tiles + tile] : 0.f;
-      const float gl = have && ga != nullptr ? ga[jl] : 1.f;
-      const float cl = sl != 0.f ? sl * gl : 0.f;
       const uint64_t rows_there = __ballot(sl != 0.f);
 #pragma unroll 4
       for (int t = 0; t < min(per, a.routes - j0); ++t) {
         const int src = (lane & ~(per - 1)) + t;
-        const float cj = __shfl(cl, src, 64);
+        const float sj = __shfl(sl, src, 64);
         float rv[8];
         load8<F16>(rrow, in && ((rows_there >> src) & 1) ? wr.local * rowb + ((j0 + t) * H + c) * 2 : kBufOOB, rv);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) r[e] = fmaf(cj, rv[e], r[e]);
+        for (int e = 0; e < 8; ++e) r[e] = fmaf(sj, rv[e], r[e]);
       }
     }
 #pragma unroll
@@ -1067,10 +1068,11 @@ namespace {
 // That kernel holds 32 rows per wave and passes every 64-pair output tile through
 // LDS with two barriers and eight dependent scale-and-store rounds per wave, which
 // cost more than its memory traffic.  16 x 65536 queries, 16 of 512 states of
-// 128 x 128: 3.4 ms there, 2.2 ms here.  What bounds it now: the 256-byte query rows
-// read and the rows written, both scattered, about 11 GB through the L2 misses at
-// 4.8 TB/s (a 1 GiB copy reaches 5.2); without the row stores 1.0 ms less, with 32
-// or 64 pairs per wave and step within 4%.
+// 128 x 128: 3.4 ms there, 2.33 ms here (2.20 without the scattered 4-byte read of
+// each pair's gate).  What bounds it now: the 256-byte query rows read and the rows
+// written, both scattered, about 11 GB through the L2 misses at 4.7 TB/s (a 1 GiB copy
+// reaches 5.2); without the row stores 1.0 ms less, with 32 or 64 pairs per wave and
+// step within 4%.
 constexpr int AL_THREADS = 512;
 constexpr int AL_WAVES = AL_THREADS / 64;
 constexpr int AL_NJ = 3;             // 16-pair columns per wave and step
@@ -1108,9 +1110,13 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
     return p + lane < p_end ? id : -1;
   };
 
-  // Pair ids (one per lane) of this wave's first 48 pairs, ids of the next.
+  const __amdgpu_buffer_rsrc_t rg = make_rsrc(a.gates + b * a.n_index, index_bytes);
+  auto load_gate = [&](int id) { return buf_load1<F32>(rg, id >= 0 ? id * 4 : kBufOOB); };
+
+  // Pair ids (one per lane) of this wave's first 48 pairs, their gates, ids of the next.
   int p0 = te.y + AL_PAIRS * w;
   int pid = load_id(p0), pid_next = load_id(p0 + AL_PAIRS * AL_WAVES);
+  float gate = load_gate(pid);
   {
     const rawl* msrc = static_cast<const rawl*>(a.mem) + (b * a.segments + te.x) * dv * dk;
     const __amdgpu_buffer_rsrc_t rm = make_rsrc(msrc, static_cast<uint32_t>(dv * dk * sizeof(rawl)));
@@ -1169,6 +1175,7 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
   while (p0 < p_end) {
     const int pn = p0 + AL_PAIRS * AL_WAVES;
     const int pid_after = load_id(pn + AL_PAIRS * AL_WAVES);
+    const float gate_next = load_gate(pid_next);
     set_q(query_of(a, pid_next));
     f32x4 acc[NI][AL_NJ];
 #pragma unroll
@@ -1200,11 +1207,14 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
 #pragma unroll
     for (int j = 0; j < AL_NJ; ++j) {
       const int pj = __shfl(pid, 16 * j + n, 64);
+      const float gj = __shfl(gate, 16 * j + n, 64);
       float m = 0.f;
 #pragma unroll
-      for (int i = 0; i < NI; ++i)
+      for (int i = 0; i < NI; ++i) {
+        acc[i][j] *= gj;
 #pragma unroll
         for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(acc[i][j][r]));
+      }
       {  // over the four lanes of the pair
         const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
         m = fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
@@ -1236,6 +1246,7 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
     p0 = pn;
     pid = pid_next;
     pid_next = pid_after;
+    gate = gate_next;
   }
 }
 
@@ -1949,6 +1960,7 @@ extern "C" int grm_hip_retrieve_fuse(const void* memories, const int64_t* indice
     RetrieveArgs a;
     init_retrieve_args(a, memories, indices, queries, rows16, workspace, batch, segments, n_query, routes, n_index,
                        value_dim, key_dim, bad_index_count);
+    a.gates = gates;
     a.scales = scales;
     if (!scaled_supported(a, mem_dtype, q_dtype)) {
       set_error("retrieve_fuse: needs bf16 queries (or f16 queries with f16 memories), 16-byte rows and "
@@ -1970,7 +1982,7 @@ extern "C" int grm_hip_retrieve_fuse(const void* memories, const int64_t* indice
   f.h = h_online;
   f.rows = reinterpret_cast<const uint16_t*>(rows16);
   f.scales = scales;
-  f.gates = gates;
+  f.all_there = 0;
   f.w = ln_weight;
   f.bias = ln_bias;
   f.out = out;

@@ -677,7 +677,7 @@ extern "C" int grm_hip_segment_retrieve_fuse(const void* memories, const int64_t
   f.h = h_online;
   f.rows = rows16;
   f.scales = scales;
-  f.gates = nullptr;  // the rows are the weighted sums
+  f.all_there = 1;
   f.w = ln_weight;
   f.bias = ln_bias;
   f.out = out;

@@ -583,6 +583,36 @@ def _retrieve_fuse_ref(mem, idx, q, gates, h, w, b, eps=1e-5):
                              eps).reshape(B, Q, H)
 
 
+@pytest.mark.parametrize("B,Q,S,R,H,K", [(2, 50, 7, 3, 128, 128), (1, 700, 2, 2, 128, 128), (2, 90, 5, 20, 64, 64),
+                                         (1, 60, 9, 4, 200, 32)])
+def test_retrieve_fuse_rounds_gated_rows(dev, B, Q, S, R, H, K):
+    """The float16 row of a pair is the row times its gate, rounded once: with one-hot queries M q is a
+    column of M, so that everything but this rounding is exact and the result is reproduced bit for
+    bit.  Few and many pairs per 128 x 128 state (output tiles, states in LDS), smaller states in LDS,
+    more routes than 16, two value tiles, gates from 1e-6 to 1, absent rows."""
+    g = torch.Generator().manual_seed(Q + H)
+    mem = torch.randn(B, S, H, K, generator=g)
+    idx = torch.randint(0, S, (B, Q, R), generator=g)
+    idx[0, 3, 1], idx[-1, 5, 0] = -1, S
+    key = torch.randint(0, K, (B, Q), generator=g)
+    q = torch.nn.functional.one_hot(key, K).to(torch.bfloat16)
+    gates = 10.0 ** (-6 * torch.rand(B, Q, R, generator=g))
+    h = torch.randn(B, Q, H, generator=g)
+    print(f"retrieve_fuse gated rows B={B} Q={Q} S={S} R={R} H={H} K={K}", flush=True)
+    out = capi.retrieve_fuse(*[t.to(dev) for t in (mem, idx, q, gates, h)]).cpu().numpy()
+    m, ix, gt = mem.numpy(), idx.numpy(), gates.numpy()
+    want = np.zeros((B, Q, H), np.float32)
+    for r in range(R):
+        there = (ix[:, :, r] >= 0) & (ix[:, :, r] < S)
+        row = m[np.arange(B)[:, None], np.where(there, ix[:, :, r], 0), :, key.numpy()] * gt[:, :, r, None]
+        for v0 in range(0, H, 128):
+            x = row[:, :, v0:v0 + 128]
+            sh = 15 - np.frexp(np.abs(x).max(-1, keepdims=True))[1]
+            x = np.ldexp(np.ldexp(x, sh).astype(np.float16).astype(np.float32), -sh)
+            want[:, :, v0:v0 + 128] += np.where(there[..., None], x, np.float32(0))
+    assert np.array_equal(out, h.numpy() + want)
+
+
 @pytest.mark.parametrize("pairs", [1, 31, 32, 33, 63, 64, 65, 96, 97, 130])
 def test_retrieve_partial_steps(dev, pairs):
     """States of 128 x 128 with few pairs each, whose last step of up to 64 pairs is empty, half
