@@ -1153,19 +1153,22 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
   const __amdgpu_buffer_rsrc_t rq =
       make_rsrc(static_cast<const rawf*>(a.queries) + b * a.n_query * dk, static_cast<uint32_t>(a.n_query * dk * 2));
   Frag8<EF> bq[AL_NJ][NSTEP];
-  int qoff[AL_NJ];  // byte offsets of this lane's part of its three pairs' queries
+  // Byte offsets of this lane's part of its three pairs' queries.  The step goes into the
+  // vector offset: the range check compares that with the resource's size less the scalar
+  // offset, which wraps where a padded step starts past the end of a single query.
+  int qoff[AL_NJ];
   auto set_q = [&](int qrow_src) {
 #pragma unroll
     for (int j = 0; j < AL_NJ; ++j) {
       const int qrow = __shfl(qrow_src, 16 * j + n, 64);
-      qoff[j] = qrow >= 0 ? (qrow * dk + 8 * g) * 2 : kBufOOB;
+      qoff[j] = qrow >= 0 ? (qrow * dk + 8 * g) * 2 : INT32_MIN;  // past every resource, as unsigned
     }
   };
   auto load_q = [&](int c) {
 #pragma unroll
     for (int j = 0; j < AL_NJ; ++j)
       bq[j][c] = __builtin_bit_cast(Frag8<EF>, __builtin_amdgcn_raw_buffer_load_b128(
-                                                   rq, 32 * c + 8 * g < dk ? qoff[j] : kBufOOB, 64 * c, 0));
+                                                   rq, (32 * c + 8 * g < dk ? qoff[j] : INT32_MIN) + 64 * c, 0, 0));
   };
   set_q(query_of(a, pid));
 #pragma unroll
