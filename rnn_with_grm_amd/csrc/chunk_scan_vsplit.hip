@@ -398,15 +398,14 @@ __global__ __launch_bounds__(kVsThreads, 1) void scan_vsplit_kernel(const ChunkF
     const __amdgpu_buffer_rsrc_t rs =
         make_rsrc(a.snapshots + (b * a.n_snap + si) * dv * dk, static_cast<uint32_t>(dv * dk * 4));
     const int G = lane & 31, h = lane >> 5;
-    // one lane offset; the row offsets 2j apart go in the scalar offset
-    const int voff = 4 * G < dk ? ((v0 + 16 * oq + h) * dk + 4 * G) * 4 : kBufOOB;
+    const int voff = ((v0 + 16 * oq + h) * dk + 4 * G) * 4;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const f32x4 v = *reinterpret_cast<const f32x4*>(M + mf_at(16 * oq + 2 * j + h, G));
       u32x4 q;
 #pragma unroll
       for (int i = 0; i < 4; ++i) q[i] = __float_as_uint(v[i]);
-      __builtin_amdgcn_raw_buffer_store_b128(q, rs, voff, 8 * dk * j, kStreamStore);
+      store_stream(rs, 4 * G < dk ? voff + 8 * dk * j : kBufOOB, q);
     }
   };
   // Every LDS operand of a step is read first, so the reads overlap one another
@@ -572,13 +571,13 @@ __global__ __launch_bounds__(kVsThreads, 1) void scan_vsplit_kernel(const ChunkF
     if constexpr (S::SO) {
       // Rows 16 vb + [8, 16) of this wave's key half, read back from the copy it has
       // just written (its own writes: no barrier needed), four rows x 256 bytes per
-      // store; the row offsets 4 and 16 apart go in the scalar offset.
+      // store.
       if (a.snap_every > 0 && (snap_phase == 0 || c + 1 == n_chunks)) {
         const float* M = Mf + ((c + 1) & 1) * S::MFB;
         const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.snapshots + (b * a.n_snap + c / a.snap_every) * dv * dk,
                                                     static_cast<uint32_t>(dv * dk * 4));
         const int G = 16 * uk + (lane & 15), q = lane >> 4;
-        const int voff = 4 * G < dk ? ((v0 + 8 + q) * dk + 4 * G) * 4 : kBufOOB;
+        const int voff = ((v0 + 8 + q) * dk + 4 * G) * 4;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int dr = 16 * (j >> 1) + 4 * (j & 1);
@@ -586,7 +585,7 @@ __global__ __launch_bounds__(kVsThreads, 1) void scan_vsplit_kernel(const ChunkF
           u32x4 qv;
 #pragma unroll
           for (int i = 0; i < 4; ++i) qv[i] = __float_as_uint(v[i]);
-          __builtin_amdgcn_raw_buffer_store_b128(qv, rs, voff, 4 * dk * dr, kStreamStore);
+          store_stream(rs, 4 * G < dk ? voff + 4 * dk * dr : kBufOOB, qv);
         }
       }
     }

@@ -252,6 +252,11 @@ __device__ __forceinline__ typename ET<E>::raw buf_load1(__amdgpu_buffer_rsrc_t 
   }
 }
 
+// A 16-byte store takes its whole offset in the vector register (scalar offset 0).
+// With a scalar register there the compiler counts no wait state between the store and
+// the next write to its data registers, and now and then a row's first dword was then
+// the one written next (seen in apply_lds_kernel; a test looks for such calls).
+
 // Four consecutive elements converted from fp32 (OOB -> dropped).
 template <class E>
 __device__ __forceinline__ void buf_store4(__amdgpu_buffer_rsrc_t r, int off, f32x4 v) {

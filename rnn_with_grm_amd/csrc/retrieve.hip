@@ -1237,9 +1237,6 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
           q[2 * h] = pack2<F16>(ldexpf(y[0], sh), ldexpf(y[1], sh));
           q[2 * h + 1] = pack2<F16>(ldexpf(y[2], sh), ldexpf(y[3], sh));
         }
-        // (the offset in the vector register: with 64 p as the scalar offset the compiler
-        // counts no wait state between the store and the next write to q, and now and
-        // then a row's first dword of 16 bytes was the next piece's)
         __builtin_amdgcn_raw_buffer_store_b128(q, rout, v0 + 32 * p + 8 * g < dv ? ro + 64 * p : kBufOOB, 0, 0);
       }
       __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ldexpf(1.f, -sh)), rscale,

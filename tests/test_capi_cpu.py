@@ -100,3 +100,27 @@ def test_other_entry_points_reject():
                                      None) == capi.EUNSUPPORTED
     assert lib.grm_hip_chunk_update_bwd(fake, fake, fake, fake, fake, fake, fake, fake, fake, fake, fake, 0, fake,
                                         1, 4, 512, 4, 0, 0, 0.9, None) == capi.EUNSUPPORTED
+
+
+def buffer_store_calls(text, width):
+    """The argument lists of the raw buffer stores of `width` in a source."""
+    for m in re.finditer(r"__builtin_amdgcn_raw_buffer_store_%s\(" % width, text):
+        args, depth = [""], 0
+        for ch in text[m.end():]:
+            if ch == "," and depth == 0:
+                args.append("")
+                continue
+            depth += (ch in "([{") - (ch in ")]}")
+            if depth < 0:
+                break
+            args[-1] += ch
+        yield [x.strip() for x in args]
+
+
+def test_wide_buffer_stores_have_no_scalar_offset():
+    """16-byte buffer stores keep their whole offset in the vector register (grm_hip_common.h): with a
+    scalar register there, no wait state separates the store from the next write to its data."""
+    csrc = HEADER.parents[1] / "rnn_with_grm_amd" / "csrc"
+    calls = [(p.name, c) for p in sorted(csrc.glob("*.h*")) for c in buffer_store_calls(p.read_text(), "b128")]
+    assert len(calls) >= 5 and all(len(c) == 5 for _, c in calls)
+    assert [x for x in calls if x[1][3] != "0"] == []
