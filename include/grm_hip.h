@@ -67,6 +67,8 @@ uint64_t grm_hip_launch_count(void);
  *             are split into time parts scanned in parallel (two launches);
  *             with less (or NULL) each sequence is scanned by one workgroup chain.
  *             Results are the same either way up to float rounding.
+ * hidden may be the values' buffer (float32; each row is written after its last read).
+ * No other output may overlap an input, and memory_out == memory is refused.
  * Limits: 1 <= key_dim <= 256 (<= 128 for float32 inputs), value_dim >= 1;
  * seq_len >= 0; batch >= 0.
  */

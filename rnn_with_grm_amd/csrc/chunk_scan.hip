@@ -753,9 +753,23 @@ extern "C" int grm_hip_chunk_update_fwd(const void* keys, const void* values, co
     set_error("chunk_update_fwd: seq_len too large");
     return GRM_HIP_EINVAL;
   }
-  // GRM_HIP_CHUNK_DV and GRM_HIP_CHUNK_PARTS ask for the walk.
-  const bool par = in_dtype == GRM_HIP_F32 && getenv("GRM_HIP_CHUNK_DV") == nullptr &&
-                   getenv("GRM_HIP_CHUNK_PARTS") == nullptr && par_direct(batch, plan.n_chunks, value_dim, key_dim);
+  // The workgroups of the chunk-parallel kernel read one another's chunks: an output in the
+  // place of an input is for the walk, where each value column has one workgroup (hidden over
+  // values), or one per part after the state pass.  GRM_HIP_CHUNK_DV and GRM_HIP_CHUNK_PARTS
+  // ask for the walk too.
+  bool par = in_dtype == GRM_HIP_F32 && par_direct(batch, plan.n_chunks, value_dim, key_dim) &&
+             getenv("GRM_HIP_CHUNK_DV") == nullptr && getenv("GRM_HIP_CHUNK_PARTS") == nullptr;
+  if (par) {
+    const int64_t kb = batch * seq_len * key_dim * 4, vb = batch * seq_len * value_dim * 4;
+    const int64_t mb = batch * value_dim * key_dim * 4;
+    const int64_t sb = snapshots != nullptr ? mb * ((seq_len + snapshot_len - 1) / snapshot_len) : 0;
+    const void* const outs[] = {hidden, memory_out, snapshots};
+    const int64_t out_b[] = {vb, mb, sb};
+    const void* const ins[] = {keys, values, queries, memory};
+    const int64_t in_bytes[] = {kb, vb, kb, mb};
+    for (int o = 0; o < 3; ++o)
+      for (int i = 0; i < 4; ++i) par = par && !ranges_overlap(outs[o], out_b[o], ins[i], in_bytes[i]);
+  }
   // Without room for the per-part states, one workgroup walks each whole sequence.
   if (plan.n_parts > 1 && (workspace == nullptr || workspace_bytes < plan.workspace_bytes ||
                            !aligned(workspace, 16))) {

@@ -294,4 +294,11 @@ namespace grmhip {
 void set_error(const char* fmt, ...);
 void count_launch();
 int check_launch(const char* what);
+
+// Whether two byte ranges share a byte (a null range shares none).
+inline bool ranges_overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return a != nullptr && b != nullptr && x < y + static_cast<uintptr_t>(b_bytes) &&
+         y < x + static_cast<uintptr_t>(a_bytes);
+}
 }  // namespace grmhip

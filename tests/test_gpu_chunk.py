@@ -317,6 +317,24 @@ def test_chunk_parallel_scan(dev, monkeypatch, shift, B, T, K, H, seg):
         assert torch.equal(snaps, snaps1) and torch.equal(snaps[:, -1], mo)
 
 
+@pytest.mark.parametrize("B,T,K,H", [(2, 200, 64, 96), (1, 512, 32, 40), (3, 64, 100, 33)])
+def test_hidden_in_the_place_of_values(dev, B, T, K, H):
+    """Short float32 sequences whose hidden rows go where the values were: the chunk-parallel kernel
+    reads other chunks' values, so these calls take the walk, whose bits are the same."""
+    k, v, q, m = make_case(B, T, K, H, torch.float32, torch.float32, seed=T)
+    rh, rm, _ = oracle_fwd(k, v, q, m, 0.97, 64)
+    kd, qd, md = k.to(dev), q.to(dev), m.to(dev)
+    print(f"hidden in the place of values B={B} T={T} K={K} H={H}", flush=True)
+    vd = v.to(dev)
+    hid1, mo1, _ = capi.chunk_update_fwd(kd, vd, qd, md, 0.97)
+    hid, mo, _ = capi.chunk_update_fwd_noalloc(kd, vd, qd, md, 0.97, hidden=vd)
+    torch.cuda.synchronize()
+    assert hid.data_ptr() == vd.data_ptr()
+    assert torch.equal(hid, hid1) and torch.equal(mo, mo1)
+    close("hidden", hid, rh, torch.float32)
+    close("memory_out", mo, rm, torch.float32)
+
+
 def test_empty_and_zero_batch(dev):
     k, v, q, m = make_case(2, 0, 16, 8, torch.float32, torch.float32)
     hid, mo, aux = torch.ops.grm_cuda.chunk_update_forward(k.to(dev), v.to(dev), q.to(dev), m.to(dev), 0.9)
