@@ -131,6 +131,10 @@ int grm_hip_chunk_update_fwd_noalloc(const void* keys, const void* values, const
  *   chunks runs in parts, by each part's adjoint at its start
  *   [batch, parts, value_dim, key_dim]; the float32 kernels', when several workgroups
  *   share a chunk, by their partial sums of grad_keys and grad_queries.
+ * For float32 inputs a gradient may take the place of the tensor it belongs to, and
+ * grad_memory that of grad_memory_out (with fewer than 8 tokens not grad_memory and the
+ * others at once: refused where it does not work).  For 16-bit inputs no output may
+ * overlap an input.
  */
 int grm_hip_chunk_update_bwd(const void* grad_hidden, const void* grad_memory_out, const void* keys,
                              const void* values, const void* queries, const void* memory,

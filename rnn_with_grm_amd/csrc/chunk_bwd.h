@@ -24,7 +24,7 @@ struct BwdGenArgs {
   void* dq_out;
   void* dk_out;
   void* dv_out;
-  void* dm_out;
+  void* dm_out;         // grad_memory, or float32 scratch that is copied there at the end
   int64_t batch;
   int64_t T;
   int dk;
@@ -33,6 +33,7 @@ struct BwdGenArgs {
   int splits;           // workgroups sharing one chunk's value tiles
   int tiles_per_split;
   int mem_f32;
+  int dm_f32;           // dm_out is float32
   int vec_k;            // dk and the gradient rows allow 4-element stores
   int vec_v;            // dv likewise
   float c;

@@ -107,7 +107,6 @@ __global__ __launch_bounds__(GNT) void bwd_outer_kernel(const BwdGenArgs a) {
   }
   if (v >= dv) return;
   if (a.n_chunks == 1) {
-    const bool f32m = a.mem_f32 != 0;
     const float decay_L = pw[L];
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt)
@@ -116,9 +115,7 @@ __global__ __launch_bounds__(GNT) void bwd_outer_kernel(const BwdGenArgs a) {
         const int k = 16 * kt + 4 * g + r;
         if (k >= dk) continue;
         const int64_t i = (b * dv + v) * dk + k;
-        const float y = fmaf(decay_L, ld_state<E>(a.dmo, i, f32m), acc[kt][r]);
-        if (f32m) static_cast<float*>(a.dm_out)[i] = y;
-        else static_cast<raw*>(a.dm_out)[i] = ET<E>::from_f(y);
+        st_state<E>(a.dm_out, i, a.dm_f32 != 0, fmaf(decay_L, ld_state<E>(a.dmo, i, a.mem_f32 != 0), acc[kt][r]));
       }
     return;
   }
@@ -142,8 +139,7 @@ __global__ __launch_bounds__(GNT) void bwd_carry_kernel(const BwdGenArgs a) {
   if (i >= a.batch * plane) return;
   const int64_t b = i / plane;
   float* slot = a.gbuf + b * a.n_chunks * plane + (i - b * plane);
-  const bool f32m = a.mem_f32 != 0;
-  float x = ld_state<E>(a.dmo, i, f32m);
+  float x = ld_state<E>(a.dmo, i, a.mem_f32 != 0);
   const float decay_c = a.pw[BCT];
   const float decay_last = a.pw[static_cast<int>(a.T - static_cast<int64_t>(a.n_chunks - 1) * BCT)];
   float buf[AHEAD];
@@ -163,8 +159,15 @@ __global__ __launch_bounds__(GNT) void bwd_carry_kernel(const BwdGenArgs a) {
       buf[j] = next >= 0 ? slot[next * plane] : 0.f;
     }
   }
-  if (f32m) static_cast<float*>(a.dm_out)[i] = x;
-  else static_cast<typename ET<E>::raw*>(a.dm_out)[i] = ET<E>::from_f(x);
+  st_state<E>(a.dm_out, i, a.dm_f32 != 0, x);
+}
+
+// grad_memory from float32 scratch, where it takes the place of an input that
+// bwd_chunk_kernel reads.
+template <class E>
+__global__ __launch_bounds__(GNT) void bwd_state_copy_kernel(const float* from, void* to, int64_t n, int f32) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * GNT + threadIdx.x;
+  if (i < n) st_state<E>(to, i, f32 != 0, from[i]);
 }
 
 template <class E, int DKP>
@@ -447,8 +450,10 @@ __global__ __launch_bounds__(GNT) void split_sum_kernel(const BwdGenArgs a) {
   }
 }
 
+// copy_to: grad_memory where a.dm_out is scratch, else NULL.
+// outer_last (one chunk): the kernel that writes grad_memory runs after the other.
 template <class E, int DKP>
-int launch_gen(const BwdGenArgs& a, hipStream_t s) {
+int launch_gen(const BwdGenArgs& a, void* copy_to, bool outer_last, hipStream_t s) {
   using S = GenShape<E, DKP>;
   if (S::lds_bytes > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_chunk_kernel<E, DKP>),
@@ -460,20 +465,33 @@ int launch_gen(const BwdGenArgs& a, hipStream_t s) {
     }
   }
   const int64_t bc = a.batch * a.n_chunks;
-  hipLaunchKernelGGL((bwd_outer_kernel<E, DKP>), dim3(static_cast<unsigned>(bc * ((a.dv + OUTER_V - 1) / OUTER_V))),
-                     dim3(GNT), 0, s, a);
-  int rc = check_launch("chunk_update_bwd(outer)");
+  const int64_t n = a.batch * a.dv * a.dk;
+  const dim3 state_grid(static_cast<unsigned>((n + GNT - 1) / GNT));
+  auto outer = [&] {
+    hipLaunchKernelGGL((bwd_outer_kernel<E, DKP>), dim3(static_cast<unsigned>(bc * ((a.dv + OUTER_V - 1) / OUTER_V))),
+                       dim3(GNT), 0, s, a);
+    return check_launch("chunk_update_bwd(outer)");
+  };
+  int rc = outer_last ? GRM_HIP_OK : outer();
   if (rc != GRM_HIP_OK) return rc;
   if (a.n_chunks > 1) {
-    const int64_t n = a.batch * a.dv * a.dk;
-    hipLaunchKernelGGL(bwd_carry_kernel<E>, dim3(static_cast<unsigned>((n + GNT - 1) / GNT)), dim3(GNT), 0, s, a);
+    hipLaunchKernelGGL(bwd_carry_kernel<E>, state_grid, dim3(GNT), 0, s, a);
     rc = check_launch("chunk_update_bwd(carry)");
     if (rc != GRM_HIP_OK) return rc;
   }
   hipLaunchKernelGGL((bwd_chunk_kernel<E, DKP>), dim3(static_cast<unsigned>(bc * a.splits)), dim3(GNT), S::lds_bytes, s,
                      a);
   rc = check_launch("chunk_update_bwd(gradients)");
-  if (rc != GRM_HIP_OK || a.splits == 1) return rc;
+  if (rc != GRM_HIP_OK) return rc;
+  if (outer_last) rc = outer();
+  if (rc != GRM_HIP_OK) return rc;
+  if (copy_to != nullptr) {
+    hipLaunchKernelGGL(bwd_state_copy_kernel<E>, state_grid, dim3(GNT), 0, s, static_cast<const float*>(a.dm_out),
+                       copy_to, n, a.mem_f32);
+    rc = check_launch("chunk_update_bwd(state copy)");
+    if (rc != GRM_HIP_OK) return rc;
+  }
+  if (a.splits == 1) return rc;
   const int64_t want = (a.batch * a.T * a.dk + GNT - 1) / GNT;
   hipLaunchKernelGGL(split_sum_kernel<E>, dim3(static_cast<unsigned>(std::min<int64_t>(want, 4096)), 2), dim3(GNT), 0,
                      s, a);
@@ -481,11 +499,11 @@ int launch_gen(const BwdGenArgs& a, hipStream_t s) {
 }
 
 template <class E>
-int launch_gen_width(const BwdGenArgs& a, hipStream_t s) {
-  if (a.dk <= 32) return launch_gen<E, 32>(a, s);
-  if (a.dk <= 64) return launch_gen<E, 64>(a, s);
-  if (a.dk <= 128) return launch_gen<E, 128>(a, s);
-  if constexpr (sizeof(typename ET<E>::raw) == 2) return launch_gen<E, 256>(a, s);
+int launch_gen_width(const BwdGenArgs& a, void* copy_to, bool outer_last, hipStream_t s) {
+  if (a.dk <= 32) return launch_gen<E, 32>(a, copy_to, outer_last, s);
+  if (a.dk <= 64) return launch_gen<E, 64>(a, copy_to, outer_last, s);
+  if (a.dk <= 128) return launch_gen<E, 128>(a, copy_to, outer_last, s);
+  if constexpr (sizeof(typename ET<E>::raw) == 2) return launch_gen<E, 256>(a, copy_to, outer_last, s);
   set_error("chunk_update_bwd: key_dim %d exceeds 128 for float32", a.dk);
   return GRM_HIP_EUNSUPPORTED;
 }
@@ -494,7 +512,33 @@ int launch_gen_width(const BwdGenArgs& a, hipStream_t s) {
 
 int launch_bwd_gen(BwdGenArgs a, int in_dtype, float* ws, int64_t floats, hipStream_t s) {
   const int64_t vtiles = (a.dv + kGenDv - 1) / kGenDv;
-  const int64_t adj = a.n_chunks > 1 ? a.batch * a.n_chunks * static_cast<int64_t>(a.dv) * a.dk : 0;
+  const int64_t state = a.batch * static_cast<int64_t>(a.dv) * a.dk;
+  int64_t adj = a.n_chunks > 1 ? a.n_chunks * state : 0;
+  // grad_memory in the place of grad_memory_out or memory, which bwd_chunk_kernel reads: it
+  // goes through scratch behind the adjoints.  From eight tokens on the documented workspace
+  // has room for that; below, grad_memory is written last, from rows that must still be there.
+  const int64_t es = in_dtype == GRM_HIP_F32 ? 4 : 2, state_b = state * (a.mem_f32 != 0 ? 4 : 2);
+  const bool in_place =
+      ranges_overlap(a.dm_out, state_b, a.dmo, state_b) || ranges_overlap(a.dm_out, state_b, a.memory, state_b);
+  void* copy_to = nullptr;
+  bool outer_last = false;
+  a.dm_f32 = a.mem_f32;
+  if (in_place && adj + state <= floats) {
+    copy_to = a.dm_out;
+    a.dm_out = ws + adj;
+    a.dm_f32 = 1;
+    adj += state;
+  } else if (in_place) {
+    outer_last = true;
+    const int64_t kb = a.batch * a.T * a.dk * es, vb = a.batch * a.T * a.dv * es;
+    const void* const outs[] = {a.dq_out, a.dk_out, a.dv_out};
+    const int64_t out_b[] = {kb, kb, vb};
+    for (int o = 0; o < 3; ++o)
+      if (ranges_overlap(outs[o], out_b[o], a.queries, kb) || ranges_overlap(outs[o], out_b[o], a.dh, vb)) {
+        set_error("chunk_update_bwd: fewer than 8 tokens with grad_memory and the rows' gradients in place");
+        return GRM_HIP_EINVAL;
+      }
+  }
   // Enough workgroups for two per CU, at least two value tiles each (a split
   // repeats the chunk's P and its dS products, worth about one tile's work), and
   // the partial sums within the workspace.
@@ -505,8 +549,8 @@ int launch_bwd_gen(BwdGenArgs a, int in_dtype, float* ws, int64_t floats, hipStr
   const int64_t per = (vtiles + splits - 1) / splits;
   a.tiles_per_split = static_cast<int>(per);
   a.splits = static_cast<int>((vtiles + per - 1) / per);
-  if (adj > floats || std::min<int64_t>(a.T, BCT) * a.dv * 4 > INT32_MAX || bc * a.splits > INT32_MAX || bc * ((a.dv + OUTER_V - 1) / OUTER_V) > INT32_MAX ||
-      (a.batch * a.dv * a.dk + GNT - 1) / GNT > INT32_MAX) {
+  if (adj > floats || std::min<int64_t>(a.T, BCT) * a.dv * 4 > INT32_MAX || bc * a.splits > INT32_MAX ||
+      bc * ((a.dv + OUTER_V - 1) / OUTER_V) > INT32_MAX || (state + GNT - 1) / GNT > INT32_MAX) {
     set_error("chunk_update_bwd: problem too large for one launch");
     return GRM_HIP_EINVAL;
   }
@@ -514,9 +558,9 @@ int launch_bwd_gen(BwdGenArgs a, int in_dtype, float* ws, int64_t floats, hipStr
   a.part_k = ws + adj;
   a.part_q = ws + adj + a.splits * rows;
   switch (in_dtype) {
-    case GRM_HIP_F32: return launch_gen_width<F32>(a, s);
-    case GRM_HIP_F16: return launch_gen_width<F16>(a, s);
-    default: return launch_gen_width<BF16>(a, s);
+    case GRM_HIP_F32: return launch_gen_width<F32>(a, copy_to, outer_last, s);
+    case GRM_HIP_F16: return launch_gen_width<F16>(a, copy_to, outer_last, s);
+    default: return launch_gen_width<BF16>(a, copy_to, outer_last, s);
   }
 }
 

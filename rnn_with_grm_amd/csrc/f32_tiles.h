@@ -68,4 +68,10 @@ __device__ __forceinline__ float ld_state(const void* p, int64_t i, bool f32) {
   return f32 ? static_cast<const float*>(p)[i] : ET<E>::to_f(static_cast<const typename ET<E>::raw*>(p)[i]);
 }
 
+template <class E>
+__device__ __forceinline__ void st_state(void* p, int64_t i, bool f32, float x) {
+  if (f32) static_cast<float*>(p)[i] = x;
+  else static_cast<typename ET<E>::raw*>(p)[i] = ET<E>::from_f(x);
+}
+
 }  // namespace grmhip

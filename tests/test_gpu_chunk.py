@@ -479,6 +479,44 @@ def test_float32_backward(dev, dtype, mem_dtype, shift, B, T, K, H):
             close_elementwise(name, x, r)
 
 
+@pytest.mark.parametrize("state_over", ["grad_memory_out", "memory"])
+@pytest.mark.parametrize("dtype,mem_dtype,B,T,K,H,rows", [
+    (torch.float32, torch.float32, 2, 300, 32, 64, True), (torch.float32, torch.float32, 1, 64, 25, 512, True),
+    (torch.float32, torch.float32, 3, 8, 16, 33, True), (torch.float32, torch.float32, 2, 3, 16, 40, False),
+    (torch.float16, torch.float16, 2, 150, 25, 40, False)])
+def test_float32_backward_in_place(dev, state_over, dtype, mem_dtype, B, T, K, H, rows):
+    """grad_memory in the place of grad_memory_out or of memory (and with `rows` every other gradient
+    in the place of its tensor): through scratch with many, one and eight tokens of one chunk, written
+    last with three, and 16-bit states of a width that the 16-bit kernels refuse.  Against the oracle
+    at the bars of test_float32_backward."""
+    k, v, q, m = make_case(B, T, K, H, dtype, mem_dtype, seed=T)
+    g = torch.Generator().manual_seed(9)
+    dh = torch.randn(B, T, H, generator=g).to(dtype)
+    dm = torch.randn(B, H, K, generator=g).to(mem_dtype)
+    ref = orc.chunk_update_bwd(*[x.double().numpy() for x in (dh, dm, k, v, q, m)], 0.97)
+    d = {n: x.to(dev) for n, x in (("dh", dh), ("dm", dm), ("k", k), ("v", v), ("q", q), ("m", m))}
+    gm = d["dm"] if state_over == "grad_memory_out" else d["m"]
+    gk, gv, gq = (d["k"], d["v"], d["q"]) if rows else [torch.empty_like(d[n]) for n in "kvq"]
+    states = torch.empty((B, (T + 63) // 64, H, K), dtype=torch.float32, device=dev)
+    partial = torch.empty((2, B, (H + 15) // 16, T, K), dtype=torch.float32, device=dev)
+
+    def call(gk, gv, gq):
+        p = [capi._ptr(x) for x in (d["dh"], d["dm"], d["k"], d["v"], d["q"], d["m"], gk, gv, gq, gm, states)]
+        return capi.load().grm_hip_chunk_update_bwd(*p, 0, capi._ptr(partial), B, T, K, H, capi.dtype_code(dtype),
+                                                    capi.dtype_code(mem_dtype), 0.97, capi._stream(d["k"]))
+
+    print(f"backward in place {state_over} {dtype} B={B} T={T} K={K} H={H}", flush=True)
+    if T < 8:  # nothing left to form grad_memory from: refused
+        assert call(gk, gv, d["q"]) == capi.EINVAL
+    assert call(gk, gv, gq) == capi.OK
+    torch.cuda.synchronize()
+    for name, x, r in zip(("grad_keys", "grad_values", "grad_queries", "grad_memory"), (gk, gv, gq, gm), ref):
+        if x.dtype == torch.float32:
+            np.testing.assert_allclose(x.double().cpu().numpy(), r, rtol=1e-5, atol=1e-5, err_msg=name)
+        else:
+            close_elementwise(name, x, r)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_segment_scan_gradient_of_one_output(dev, dtype):
     """cuda_segment_scan when only one of its two differentiable outputs enters the loss (the other's
