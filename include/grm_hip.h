@@ -135,6 +135,9 @@ int grm_hip_chunk_update_fwd_noalloc(const void* keys, const void* values, const
  * grad_memory that of grad_memory_out (with fewer than 8 tokens not grad_memory and the
  * others at once: refused where it does not work).  For 16-bit inputs no output may
  * overlap an input.
+ * Infinities and NaN: with float32 inputs, and no gradient over values or grad_hidden, a
+ * token's reach only the gradients that depend on it; otherwise also others of its block
+ * of 16 tokens.
  */
 int grm_hip_chunk_update_bwd(const void* grad_hidden, const void* grad_memory_out, const void* keys,
                              const void* values, const void* queries, const void* memory,

@@ -34,6 +34,7 @@ struct BwdGenArgs {
   int tiles_per_split;
   int mem_f32;
   int dm_f32;           // dm_out is float32
+  int exact;            // infinities and NaN kept to the gradients that depend on them
   int vec_k;            // dk and the gradient rows allow 4-element stores
   int vec_v;            // dv likewise
   float c;

@@ -344,6 +344,12 @@ __global__ __launch_bounds__(GNT) void bwd_chunk_kernel(const BwdGenArgs a) {
     __syncthreads();  // P read: the region takes the value tiles
   }
 
+  // NaN once a result is not finite
+  float check = 0.f;
+  auto finite = [&](f32x4 x) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) check = fmaf(x[r], 0.f, check);
+  };
   f32x4 dsacc[4], dq[KT], dkk[KT];
 #pragma unroll
   for (int jb = 0; jb < 4; ++jb) dsacc[jb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -388,6 +394,7 @@ __global__ __launch_bounds__(GNT) void bwd_chunk_kernel(const BwdGenArgs a) {
 #pragma unroll
       for (int ib = 0; ib < 4; ++ib)
         if (ib >= w) acc = mfma4(lds_col4<E>(Hs + (16 * ib + 4 * g) * GVS + 16 * vb + n, GVS), pT[ib], acc);
+      finite(acc);
       const int v = vt * kGenDv + 16 * vb + 4 * g;
       out4<E>(rdv, jrow * dv + v, dv - v, a.vec_v != 0, acc);
     }
@@ -422,6 +429,8 @@ __global__ __launch_bounds__(GNT) void bwd_chunk_kernel(const BwdGenArgs a) {
       if (xb <= w) aq = mfma4(lds_col4<E>(Ks + o, KS), dsacc[xb], aq);
       if (xb >= w) ak = mfma4(lds_col4<E>(Qs + o, KS), dsT[xb], ak);
     }
+    finite(aq);
+    finite(ak);
     const int k = 16 * kt + 4 * g;
     if (partial) {
       out4<F32>(rqo, jrow * dk + k, dk - k, a.vec_k != 0, aq);
@@ -430,6 +439,84 @@ __global__ __launch_bounds__(GNT) void bwd_chunk_kernel(const BwdGenArgs a) {
       out4<E>(rqo, jrow * dk + k, dk - k, a.vec_k != 0, aq);
       out4<E>(rko, jrow * dk + k, dk - k, a.vec_k != 0, ak);
     }
+  }
+  if (a.exact == 0 || !__any(check != check)) return;
+
+  // ---- Some result of this wave's tokens is not finite.  The products above multiply the
+  // zeros above the diagonal too, and zero times an infinity or NaN is NaN: a token's would
+  // reach the gradients of its whole 16-token block.  The wave's rows once more, one product
+  // at a time and only those that belong to a gradient.  Lane (g, n): token 16w + n, columns
+  // 8g .. 8g + 7 of every 32.  dQ and dK first: dS is in LDS.
+  const __amdgpu_buffer_rsrc_t rm = make_rsrc(msrc, static_cast<uint32_t>(dv * dk * (m32 ? 4 : ES)));
+  const __amdgpu_buffer_rsrc_t rg = make_rsrc(gsrc, static_cast<uint32_t>(dv * dk * (g32 ? 4 : ES)));
+  const int v_begin = vt_begin * kGenDv, v_end = min(vt_end * kGenDv, dv);
+#pragma unroll 1
+  for (int k0 = 8 * g; k0 < DKP; k0 += 32) {
+    float aq[8], ak[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) aq[e] = ak[e] = 0.f;
+#pragma unroll 1
+    for (int v = v_begin; v < v_end; ++v) {
+      const float hx = ET<E>::to_f(buf_load1<E>(rh, (jrow * dv + v) * ES));  // zero from token L on
+      const float vx = ET<E>::to_f(buf_load1<E>(rv, (jrow * dv + v) * ES));
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        aq[e] = fmaf(hx, ld_mem(rm, v * dk + k0 + e, m32, k0 + e < dk, E()), aq[e]);
+        ak[e] = fmaf(vx, ld_mem(rg, v * dk + k0 + e, g32, k0 + e < dk, E()), ak[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      aq[e] *= sq;
+      ak[e] *= wl;
+    }
+#pragma unroll 1
+    for (int x = 0; x < L; ++x) {
+      const float dsq = Ps[jrow * GPS + x], dsk = Ps[x * GPS + jrow];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (x <= jrow) aq[e] = fmaf(dsq, ET<E>::to_f(Ks[x * KS + k0 + e]), aq[e]);
+        if (x >= jrow) ak[e] = fmaf(dsk, ET<E>::to_f(Qs[x * KS + k0 + e]), ak[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int off = jrow < L && k0 + e < dk ? jrow * dk + k0 + e : -1;
+      if (partial) {
+        buf_store1<F32>(rqo, off >= 0 ? off * 4 : kBufOOB, aq[e]);
+        buf_store1<F32>(rko, off >= 0 ? off * 4 : kBufOOB, ak[e]);
+      } else {
+        buf_store1<E>(rqo, off >= 0 ? off * ES : kBufOOB, aq[e]);
+        buf_store1<E>(rko, off >= 0 ? off * ES : kBufOOB, ak[e]);
+      }
+    }
+  }
+#pragma unroll 1
+  for (int v0 = v_begin + 8 * g; v0 < v_end; v0 += 32) {
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < dk; ++k) {
+      const float kx = ET<E>::to_f(Ks[jrow * KS + k]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = fmaf(ld_mem(rg, (v0 + e) * dk + k, g32, v0 + e < dv, E()), kx, acc[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] *= wl;
+#pragma unroll 1
+    for (int i = jrow; i < L; ++i) {
+      float p = 0.f;
+#pragma unroll 1
+      for (int k = 0; k < dk; ++k) p = fmaf(ET<E>::to_f(Qs[i * KS + k]), ET<E>::to_f(Ks[jrow * KS + k]), p);
+      p *= c * pw[i - jrow];
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        acc[e] = fmaf(ET<E>::to_f(buf_load1<E>(rh, v0 + e < dv ? (i * dv + v0 + e) * ES : kBufOOB)), p, acc[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      buf_store1<E>(rdv, jrow < L && v0 + e < dv ? (jrow * dv + v0 + e) * ES : kBufOOB, acc[e]);
   }
 }
 
@@ -518,6 +605,9 @@ int launch_bwd_gen(BwdGenArgs a, int in_dtype, float* ws, int64_t floats, hipStr
   // goes through scratch behind the adjoints.  From eight tokens on the documented workspace
   // has room for that; below, grad_memory is written last, from rows that must still be there.
   const int64_t es = in_dtype == GRM_HIP_F32 ? 4 : 2, state_b = state * (a.mem_f32 != 0 ? 4 : 2);
+  const int64_t kb = a.batch * a.T * a.dk * es, vb = a.batch * a.T * a.dv * es;
+  const void* const outs[] = {a.dq_out, a.dk_out, a.dv_out};
+  const int64_t out_b[] = {kb, kb, vb};
   const bool in_place =
       ranges_overlap(a.dm_out, state_b, a.dmo, state_b) || ranges_overlap(a.dm_out, state_b, a.memory, state_b);
   void* copy_to = nullptr;
@@ -530,9 +620,6 @@ int launch_bwd_gen(BwdGenArgs a, int in_dtype, float* ws, int64_t floats, hipStr
     adj += state;
   } else if (in_place) {
     outer_last = true;
-    const int64_t kb = a.batch * a.T * a.dk * es, vb = a.batch * a.T * a.dv * es;
-    const void* const outs[] = {a.dq_out, a.dk_out, a.dv_out};
-    const int64_t out_b[] = {kb, kb, vb};
     for (int o = 0; o < 3; ++o)
       if (ranges_overlap(outs[o], out_b[o], a.queries, kb) || ranges_overlap(outs[o], out_b[o], a.dh, vb)) {
         set_error("chunk_update_bwd: fewer than 8 tokens with grad_memory and the rows' gradients in place");
@@ -554,6 +641,10 @@ int launch_bwd_gen(BwdGenArgs a, int in_dtype, float* ws, int64_t floats, hipStr
     set_error("chunk_update_bwd: problem too large for one launch");
     return GRM_HIP_EINVAL;
   }
+  // bwd_chunk_kernel may read values and grad_hidden again after it has written gradients.
+  a.exact = static_cast<int64_t>(a.dv) * a.dk * 4 <= INT32_MAX;
+  for (int o = 0; o < 3; ++o)
+    if (ranges_overlap(outs[o], out_b[o], a.values, vb) || ranges_overlap(outs[o], out_b[o], a.dh, vb)) a.exact = 0;
   a.gbuf = ws;
   a.part_k = ws + adj;
   a.part_q = ws + adj + a.splits * rows;

@@ -479,6 +479,36 @@ def test_float32_backward(dev, dtype, mem_dtype, shift, B, T, K, H):
             close_elementwise(name, x, r)
 
 
+@pytest.mark.parametrize("dtype,B,T,K,H", [(torch.float32, 2, 150, 32, 64), (torch.float32, 1, 64, 64, 512),
+                                           (torch.float32, 1, 90, 100, 33), (torch.float16, 2, 130, 25, 40)])
+def test_float32_backward_non_finite(dev, dtype, B, T, K, H):
+    """An infinite element of grad_hidden, a NaN in keys, an infinite one in queries and a NaN in
+    values: exactly the gradients that depend on them are not finite (the oracle goes token by token),
+    the others within the bars of test_float32_backward."""
+    k, v, q, m = make_case(B, T, K, H, dtype, torch.float32, seed=T)
+    g = torch.Generator().manual_seed(9)
+    dh = torch.randn(B, T, H, generator=g).to(dtype)
+    dm = torch.randn(B, H, K, generator=g)
+    inf = float("inf")
+    for x, t, c, bad in ((dh, 5, 3, inf), (k, 37, 2, float("nan")), (q, 22, 1, -inf), (v, 61, 4, float("nan")),
+                         (dh, T - 9, 7, -inf)):
+        y = x.clone()
+        y[-1, t, c] = bad
+        args = [y if z is x else z for z in (dh, dm, k, v, q, m)]
+        print(f"float32 backward non-finite {dtype} B={B} T={T} K={K} H={H} token {t}", flush=True)
+        got = capi.chunk_update_bwd(*[z.to(dev) for z in args], 0.97)
+        torch.cuda.synchronize()
+        ref = orc.chunk_update_bwd(*[z.double().numpy() for z in args], 0.97)
+        for name, z, r in zip(("grad_keys", "grad_values", "grad_queries", "grad_memory"), got, ref):
+            z = z.cpu()
+            fin = np.isfinite(r)
+            assert np.array_equal(torch.isfinite(z).numpy(), fin), (name, t)
+            if z.dtype == torch.float32:
+                np.testing.assert_allclose(z.double().numpy()[fin], r[fin], rtol=1e-5, atol=1e-5, err_msg=name)
+            else:
+                close_elementwise(name, z[torch.from_numpy(fin)], r[fin])
+
+
 @pytest.mark.parametrize("state_over", ["grad_memory_out", "memory"])
 @pytest.mark.parametrize("dtype,mem_dtype,B,T,K,H,rows", [
     (torch.float32, torch.float32, 2, 300, 32, 64, True), (torch.float32, torch.float32, 1, 64, 25, 512, True),
