@@ -389,15 +389,17 @@ def close_elementwise(name, got, ref, rtol=2e-2, atol=2e-3):
                                              (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16)])
 @pytest.mark.parametrize("B,T,K,H", [(2, 300, 128, 128), (3, 129, 64, 64), (1, 640, 96, 96), (2, 64, 128, 32),
                                      (1, 7, 128, 32), (1, 12, 128, 32), (2, 200, 32, 64), (1, 200, 64, 512),
-                                     (1, 2000, 64, 512), (2, 1000, 64, 96)])
+                                     (1, 2000, 64, 512), (2, 1000, 64, 96), (96, 70, 128, 96), (200, 70, 64, 32)])
 def test_mfma_backward(dev, monkeypatch, dtype, mem_dtype, B, T, K, H):
     """The chunk-parallel MFMA backward (16-bit inputs, value_dim a multiple of 32: the adjoint
     pass, then the per-chunk gradients over every value tile) against the double-precision
-    oracle and against the scalar per-token kernel (GRM_HIP_BWD_MFMA=0), element by element at
+    oracle and against the float32 kernels (GRM_HIP_BWD_MFMA=0), element by element at
     rtol 2e-2 / atol 2e-3: ragged last chunks, key widths below the padded 64/128, one to
-    sixteen value tiles, a half-filled 64-row adjoint tile (96 values), one chunk (12 tokens),
-    7 tokens, where the adjoint buffer would not fit the workspace and the scalar kernel runs,
-    and adjoint walks split into 2, 4 and 8 parts (640, 1000 and 2000 tokens)."""
+    sixteen value tiles, one chunk (12 tokens), 7 tokens, where the adjoint buffer would not
+    fit the workspace and the float32 kernels run, and adjoint walks split into 2, 4 and 8
+    parts (640, 1000 and 2000 tokens).  All of these walk 32 value rows per workgroup; the
+    two with 192 and 200 workgroups of 64 rows walk those, with half-filled ones (96 and 32
+    values), in one part that writes grad_memory itself."""
     k, v, q, m = make_case(B, T, K, H, dtype, mem_dtype, seed=B * 13 + T)
     g = torch.Generator().manual_seed(7)
     dh = torch.randn(B, T, H, generator=g).to(dtype)
@@ -406,14 +408,14 @@ def test_mfma_backward(dev, monkeypatch, dtype, mem_dtype, B, T, K, H):
     print(f"mfma backward B={B} T={T} K={K} H={H} {dtype} state {mem_dtype}", flush=True)
     got = capi.chunk_update_bwd(*args, 0.97)
     monkeypatch.setenv("GRM_HIP_BWD_MFMA", "0")
-    scalar = capi.chunk_update_bwd(*args, 0.97)
+    f32 = capi.chunk_update_bwd(*args, 0.97)
     torch.cuda.synchronize()
     ref = orc.chunk_update_bwd(dh.double().numpy(), dm.double().numpy(), k.double().numpy(), v.double().numpy(),
                                q.double().numpy(), m.double().numpy(), 0.97)
-    for name, x, y, r in zip(("grad_keys", "grad_values", "grad_queries", "grad_memory"), got, scalar, ref):
+    for name, x, y, r in zip(("grad_keys", "grad_values", "grad_queries", "grad_memory"), got, f32, ref):
         assert torch.isfinite(x.float()).all(), name
         close_elementwise(name, x, r)
-        close_elementwise(name + " vs scalar kernel", x, y.float().cpu().double().numpy())
+        close_elementwise(name + " vs float32 kernels", x, y.float().cpu().double().numpy())
 
 
 @pytest.mark.parametrize("B,T,K,H,mem_dtype", [(1, 2000, 64, 512, torch.float32), (2, 1000, 64, 96, torch.bfloat16),

@@ -645,8 +645,7 @@ def test_retrieve_fuse_states_in_lds(dev, mem_dtype, q_dtype, B, Q, S, R, H, K):
     """retrieve_fuse where a state is kept in LDS for many pairs: fewer pairs than a wave takes,
     one more than one and than eight waves take (48, 384), value widths of every padded size with
     partial tiles, key widths below the padded ones, a single query that ends before the last padded
-    key step begins, several work tiles per state, sorts over one workgroup and over several (65536
-    pairs on); states of very different magnitude, and pairs with
+    key step begins, sorts over one workgroup and over several (65536 pairs on); states of very different magnitude, and pairs with
     an invalid index whose gate is NaN (absent, whatever its gate).  Rows are kept as float16 scaled
     by their largest value: 2^-11 of it each, R of them summed under gates that add to one, before
     a LayerNorm of unit scale, so 2e-3 of the output's largest value bounds the error."""
@@ -672,6 +671,29 @@ def test_retrieve_fuse_states_in_lds(dev, mem_dtype, q_dtype, B, Q, S, R, H, K):
     assert torch.equal(out, again)
     got = out.double().cpu().numpy()
     assert np.abs(got - ref).max() <= 2e-3 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("S,H,K", [(40, 128, 128), (40, 64, 64), (300, 128, 128)])
+def test_retrieve_fuse_skewed_selection(dev, S, H, K):
+    """60% of 12000 pairs choose one state: its list spans many work tiles, the last of them no
+    multiple of the 48 pairs of a wave, the 384 of a workgroup or 64, in the kernel with states in LDS
+    (300 pairs per state on average, or a small state) and in the one with output tiles (40 per
+    state).  Bound as in test_retrieve_fuse_states_in_lds."""
+    g = torch.Generator().manual_seed(S + H)
+    mem = torch.randn(1, S, H, K, generator=g) * 0.3
+    idx = torch.randint(0, S, (1, 3000, 4), generator=g)
+    idx[torch.rand(1, 3000, 4, generator=g) < 0.6] = 0
+    n0 = int((idx == 0).sum())
+    assert n0 > 7000 and (n0 % 512) % 48 != 0 and (n0 % 512) % 64 != 0
+    q = norm(torch.randn(1, 3000, K, generator=g)).to(torch.bfloat16)
+    gates = torch.softmax(torch.randn(1, 3000, 4, generator=g), dim=-1)
+    h = torch.randn(1, 3000, H, generator=g)
+    w, b = 1 + 0.1 * torch.randn(H, generator=g), 0.1 * torch.randn(H, generator=g)
+    print(f"retrieve_fuse skewed S={S} H={H} K={K}", flush=True)
+    out = capi.retrieve_fuse(*[t.to(dev) for t in (mem, idx, q, gates, h, w, b)])
+    torch.cuda.synchronize()
+    ref = _retrieve_fuse_ref(mem, idx, q, gates, h, w, b)
+    assert np.abs(out.double().cpu().numpy() - ref).max() <= 2e-3 * np.abs(ref).max()
 
 
 @pytest.mark.parametrize("mem_dtype", [torch.float32, torch.float16, torch.bfloat16])
