@@ -19,6 +19,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "grm_hip.h"
@@ -37,7 +38,6 @@ constexpr int64_t kMaxSegments = 16384;
 constexpr int AP_THREADS = 256;      // apply kernel: 4 waves
 constexpr int AP_V = kScaledTile;    // value rows per workgroup
 constexpr int AP_N = 64;             // (q, r) pairs per tile
-constexpr int kLdsApplyPairs = 256;  // see launch_scaled_rows
 
 struct RetrieveArgs {
   const void* mem;
@@ -72,7 +72,7 @@ struct RetrieveArgs {
   // gather_apply.
   const float* gates;  // [batch, n_index]
   float* scales;       // [batch, n_index, v_tiles]
-  int mean_pairs;  // pairs per segment, evenly spread
+  int lds_rows;  // apply_lds_kernel makes the scaled rows
   int out_row;         // elements per output row (dv; dk for the queries' gradient)
 };
 
@@ -313,15 +313,19 @@ __global__ __launch_bounds__(BK_THREADS) void tile_list_kernel(const RetrieveArg
   const int64_t S = a.segments;
   const int32_t* off = a.offsets + b * (S + 1);
   const int tp = a.tile_pairs;
-  for (int64_t s = tid; s < S; s += BK_THREADS) hist[s] = (off[s + 1] - off[s] + tp - 1) / tp;
+  for (int64_t s = tid; s < S; s += BK_THREADS)
+    hist[s] = static_cast<int>((static_cast<uint32_t>(off[s + 1] - off[s]) + tp - 1u) / static_cast<uint32_t>(tp));
   __syncthreads();
   int32_t* base = a.tile_base + b * (S + 1);
   bucket_offsets(hist, S, base);
   int4* tl = a.tiles + b * a.tb_max;
   for (int64_t s = tid; s < S; s += BK_THREADS) {
-    const int p0 = off[s], p1 = off[s + 1];
-    int slot = hist[s];
-    for (int p = p0; p < p1; p += tp) tl[slot++] = make_int4(static_cast<int>(s), p, min(p1, p + tp), 0);
+    int p = off[s], slot = hist[s];
+    for (int left = off[s + 1] - p; left > 0; left -= tp) {
+      const int take = min(left, tp);
+      tl[slot++] = make_int4(static_cast<int>(s), p, p + take, 0);
+      p += take;
+    }
   }
   if (tid == 0) a.n_tiles[b] = base[S];
 }
@@ -1274,12 +1278,18 @@ int launch_apply_lds(const RetrieveArgs& a, hipStream_t s) {
 // staging nothing hides: from 256 pairs per state on (128 x 128 float32 states, 64
 // pairs 460 -> 606 us, 128 pairs 222 -> 239, 256 pairs 351 -> 347, 512 pairs 604 -> 555).
 // The buffer offsets of that kernel are 32 bits.
+constexpr int kLdsApplyPairs = 256;
+
+bool rows_in_lds(const RetrieveArgs& a, int parts, int64_t tiles) {
+  const int steps = a.dk <= 32 ? 1 : a.dk <= 64 ? 2 : 4, row_blocks = a.dv <= 32 ? 2 : a.dv <= 64 ? 4 : 8;
+  const bool shared = parts * steps * row_blocks <= 48;  // fragments of 1 KB
+  return (shared || a.n_index >= kLdsApplyPairs * a.segments) && a.n_index * a.dv * 2 <= INT32_MAX &&
+         tiles * a.v_tiles * AL_THREADS <= UINT32_MAX;
+}
+
 template <class EL, class EQ, int DKP, class EF, int NPART, int NI>
 int launch_scaled_rows(const RetrieveArgs& a, hipStream_t s) {
-  constexpr bool kShared = NPART * (DKP / 32) * NI <= 48;  // fragments of 1 KB
-  if ((kShared || a.mean_pairs >= kLdsApplyPairs) && a.n_index * a.dv * 2 <= INT32_MAX &&
-      static_cast<int64_t>(a.tb_max) * a.v_tiles * AL_THREADS <= UINT32_MAX)
-    return launch_apply_lds<EL, EQ, DKP, EF, NPART, NI>(a, s);
+  if (a.lds_rows != 0) return launch_apply_lds<EL, EQ, DKP, EF, NPART, NI>(a, s);
   return launch_apply_mfma16<EL, F32, EQ, DKP, EF, NPART, true>(a, s);
 }
 
@@ -1321,6 +1331,20 @@ bool scaled_supported(const RetrieveArgs& a, int mem_dtype, int q_dtype) {
     case GRM_HIP_F32: return scaled_ok_q<F32>(a, q_dtype);
     case GRM_HIP_F16: return scaled_ok_q<F16>(a, q_dtype);
     default: return scaled_ok_q<BF16>(a, q_dtype);
+  }
+}
+
+// Exact 16-bit parts of a stored state under the scaled apply's plan.
+template <class EL>
+int scaled_parts_q(int q_dtype) {
+  return q_dtype == GRM_HIP_F16 ? MfmaPlan<EL, F32, F16>::parts : MfmaPlan<EL, F32, BF16>::parts;
+}
+
+int scaled_parts(int mem_dtype, int q_dtype) {
+  switch (mem_dtype) {
+    case GRM_HIP_F32: return scaled_parts_q<F32>(q_dtype);
+    case GRM_HIP_F16: return scaled_parts_q<F16>(q_dtype);
+    default: return scaled_parts_q<BF16>(q_dtype);
   }
 }
 
@@ -1749,20 +1773,26 @@ int64_t partial_bytes(int64_t batch, int64_t segments, int64_t n_index) {
   return c > 1 ? (batch * c * segments * 4 + 15) / 16 * 16 : 0;
 }
 
-// Pairs per apply work tile: one and a half times the mean pairs per segment (at
-// least 512, a multiple of the 64-pair MFMA tile), so balanced selections keep one
-// tile per segment and a heavily selected segment is split.  At the mean itself
-// half of the segments had a second tile of a few pairs that read the state again
-// (16 x 65536 queries over 512 states: 3.97 -> 3.67 ms).
-int64_t tile_pairs_for(int64_t segments, int64_t n_index) {
+// Pairs per apply work tile: the mean pairs per segment (at least 512, a
+// multiple of the 64-pair MFMA tile), so balanced selections keep about one
+// tile per segment and a heavily selected segment is split.  With few states
+// the longest tile is the kernel's time: at one and a half times the mean, an
+// uneven selection (weights 1 / sqrt(rank)) over 6 to 32 states took gather_apply
+// and its gradients 1.2 to 1.45 times as long (20000 queries, 2 of 6 states of
+// 128 x 128, float16: 386 -> 554 us), an even one the same.
+// `spread` (the scaled rows with states in LDS, which stage a state per tile):
+// one and a half times the mean, since at the mean half of the segments have a
+// second tile of a few pairs (16 x 65536 queries over 512 states: 3.97 -> 3.67 ms).
+// At most 2^20 pairs, so that no 32-bit count of the tiles overflows.
+int64_t tile_pairs_for(int64_t segments, int64_t n_index, bool spread = false) {
   const int64_t mean = segments > 0 ? (n_index + segments - 1) / segments : n_index;
-  const int64_t tp = (mean + mean / 2 + AP_N - 1) / AP_N * AP_N;
-  return tp > 8 * AP_N ? tp : 8 * AP_N;
+  const int64_t tp = (mean + (spread ? mean / 2 : 0) + AP_N - 1) / AP_N * AP_N;
+  return std::min<int64_t>(std::max<int64_t>(tp, 8 * AP_N), 1 << 20);
 }
 
 // Tiles per sequence at most: sum_s ceil(c_s / tp) <= n_index / tp + segments.
-int64_t tiles_max(int64_t segments, int64_t n_index) {
-  const int64_t tp = tile_pairs_for(segments, n_index);
+int64_t tiles_max(int64_t segments, int64_t n_index, bool spread = false) {
+  const int64_t tp = tile_pairs_for(segments, n_index, spread);
   return (n_index + tp - 1) / tp + segments;
 }
 
@@ -1812,7 +1842,6 @@ void init_retrieve_args(RetrieveArgs& a, const void* memories, const int64_t* in
   a.n_index = n_index;
   a.dv = static_cast<int>(hidden_size);
   a.dk = static_cast<int>(key_dim);
-  a.mean_pairs = static_cast<int>(segments > 0 ? n_index / segments : n_index);
   a.out_row = a.dv;
   a.v_tiles = static_cast<int>((hidden_size + AP_V - 1) / AP_V);
 }
@@ -1967,7 +1996,13 @@ extern "C" int grm_hip_retrieve_fuse(const void* memories, const int64_t* indice
                 "16-byte aligned memories and queries");
       return GRM_HIP_EUNSUPPORTED;
     }
-    int rc = launch_bucket<F16>(a, s);  // invalid pairs: zero rows and zero scales
+    const int64_t spread_tiles = tiles_max(segments, n_index, true);  // not more than the workspace holds
+    if (rows_in_lds(a, scaled_parts(mem_dtype, q_dtype), spread_tiles)) {
+      a.lds_rows = 1;
+      a.tile_pairs = static_cast<int>(tile_pairs_for(segments, n_index, true));
+      a.tb_max = static_cast<int>(spread_tiles);
+    }
+    int rc = launch_bucket<F16>(a, s);  // invalid pairs: zero scales
     if (rc != GRM_HIP_OK) return rc;
     if (segments > 0) {
       switch (mem_dtype) {

@@ -35,6 +35,21 @@ def test_workspace_query():
     assert ws > 0 and ws % (16 * 128 * 128 * 4) == 0
 
 
+@pytest.mark.parametrize("segments,pairs", [(1, 2**31 - 1), (3, 2**31 - 1), (1, 3 * 2**20 + 5), (7, 4000), (512, 2**20)])
+def test_gather_apply_workspace_holds_its_work_tiles(segments, pairs):
+    """The workspace of the pair sort has 16 bytes for every work tile that a selection can need: tiles
+    of the mean pairs per state, of at least 512 and at most 2^20 (so that no count of a tile's end
+    passes 32 bits)."""
+    def a16(n):
+        return (n + 15) // 16 * 16
+
+    tile = min(max(-(-(-(-pairs // segments)) // 64) * 64, 512), 2**20)
+    groups = -(-pairs // 16384) if pairs >= 65536 else 1
+    need = (a16(4 * (segments + 1)) * 2 + a16(4 * pairs) + (a16(4 * groups * segments) if groups > 1 else 0) +
+            16 * (-(-pairs // tile) + segments) + 16)
+    assert capi.load().grm_hip_gather_apply_workspace(1, segments, pairs) == need
+
+
 def test_abi_version_and_counters():
     lib = capi.load()
     assert lib.grm_hip_abi_version() == 109
