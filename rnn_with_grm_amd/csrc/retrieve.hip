@@ -1157,22 +1157,22 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
   const __amdgpu_buffer_rsrc_t rq =
       make_rsrc(static_cast<const rawf*>(a.queries) + b * a.n_query * dk, static_cast<uint32_t>(a.n_query * dk * 2));
   Frag8<EF> bq[AL_NJ][NSTEP];
-  // Byte offsets of this lane's part of its three pairs' queries.  The step goes into the
-  // vector offset: the range check compares that with the resource's size less the scalar
-  // offset, which wraps where a padded step starts past the end of a single query.
+  // Byte offsets of this lane's part of its three pairs' queries; the step is the scalar
+  // offset, which rows_in_lds keeps below the resource's size (the range check compares
+  // the vector offset with the size less the scalar offset).
   int qoff[AL_NJ];
   auto set_q = [&](int qrow_src) {
 #pragma unroll
     for (int j = 0; j < AL_NJ; ++j) {
       const int qrow = __shfl(qrow_src, 16 * j + n, 64);
-      qoff[j] = qrow >= 0 ? (qrow * dk + 8 * g) * 2 : INT32_MIN;  // past every resource, as unsigned
+      qoff[j] = qrow >= 0 ? (qrow * dk + 8 * g) * 2 : kBufOOB;
     }
   };
   auto load_q = [&](int c) {
 #pragma unroll
     for (int j = 0; j < AL_NJ; ++j)
       bq[j][c] = __builtin_bit_cast(Frag8<EF>, __builtin_amdgcn_raw_buffer_load_b128(
-                                                   rq, (32 * c + 8 * g < dk ? qoff[j] : INT32_MIN) + 64 * c, 0, 0));
+                                                   rq, 32 * c + 8 * g < dk ? qoff[j] : kBufOOB, 64 * c, 0));
   };
   set_q(query_of(a, pid));
 #pragma unroll
@@ -1272,19 +1272,19 @@ int launch_apply_lds(const RetrieveArgs& a, hipStream_t s) {
   return check_launch("retrieve_fuse(apply)");
 }
 
-// The state in LDS wherever several workgroups share a CU (up to 48 KB of parts:
-// 4 x 4000 queries, 8 of 63 states of 512 x 64, 147 -> 121 us; 8 x 2000, 8 of 200 of
-// 64 x 64, 57 -> 47 us).  Larger states leave one or two workgroups per CU, whose
-// staging nothing hides: from 256 pairs per state on (128 x 128 float32 states, 64
-// pairs 460 -> 606 us, 128 pairs 222 -> 239, 256 pairs 351 -> 347, 512 pairs 604 -> 555).
-// The buffer offsets of that kernel are 32 bits.
-constexpr int kLdsApplyPairs = 256;
-
-bool rows_in_lds(const RetrieveArgs& a, int parts, int64_t tiles) {
-  const int steps = a.dk <= 32 ? 1 : a.dk <= 64 ? 2 : 4, row_blocks = a.dv <= 32 ? 2 : a.dv <= 64 ? 4 : 8;
-  const bool shared = parts * steps * row_blocks <= 48;  // fragments of 1 KB
-  return (shared || a.n_index >= kLdsApplyPairs * a.segments) && a.n_index * a.dv * 2 <= INT32_MAX &&
-         tiles * a.v_tiles * AL_THREADS <= UINT32_MAX;
+// The state in LDS where enough pairs share its staging, which eight waves do while with
+// few pairs only one or two of them have any.  Time of the call with output tiles over
+// time with the state in LDS, 16 x 256 states, 8 routes, at 8, 32, 64, 128, 256 and 512
+// pairs per state (float32 and float16 states, widths of 32, 64 and 128 keys):
+//   32 values:   1.0-1.2, 1.1-1.3, 1.3-1.5, 1.4-1.7, 1.5-2.1, 1.4-2.2: always
+//   64 values:   0.8-1.0, 1.0-1.1, 1.1-1.3, 1.2-1.5, 1.3-1.5, 1.2-1.7: from 32 pairs
+//   128 values:  0.6-0.8, 0.7-0.9, 0.8-1.0, 0.9-1.0, 1.0-1.1, 1.1-1.4: from 256 pairs
+// The byte offsets of that kernel are 32 bits, and its scalar offsets stay inside the queries.
+bool rows_in_lds(const RetrieveArgs& a, int64_t tiles) {
+  const int64_t pairs = a.dv <= 32 ? 0 : a.dv <= 64 ? 32 : 256;
+  const int steps = a.dk <= 32 ? 1 : a.dk <= 64 ? 2 : 4;
+  return a.n_index >= pairs * a.segments && a.n_query * a.dk * 2 >= 64 * steps &&
+         a.n_index * a.dv * 2 <= INT32_MAX && tiles * a.v_tiles * AL_THREADS <= UINT32_MAX;
 }
 
 template <class EL, class EQ, int DKP, class EF, int NPART, int NI>
@@ -1331,20 +1331,6 @@ bool scaled_supported(const RetrieveArgs& a, int mem_dtype, int q_dtype) {
     case GRM_HIP_F32: return scaled_ok_q<F32>(a, q_dtype);
     case GRM_HIP_F16: return scaled_ok_q<F16>(a, q_dtype);
     default: return scaled_ok_q<BF16>(a, q_dtype);
-  }
-}
-
-// Exact 16-bit parts of a stored state under the scaled apply's plan.
-template <class EL>
-int scaled_parts_q(int q_dtype) {
-  return q_dtype == GRM_HIP_F16 ? MfmaPlan<EL, F32, F16>::parts : MfmaPlan<EL, F32, BF16>::parts;
-}
-
-int scaled_parts(int mem_dtype, int q_dtype) {
-  switch (mem_dtype) {
-    case GRM_HIP_F32: return scaled_parts_q<F32>(q_dtype);
-    case GRM_HIP_F16: return scaled_parts_q<F16>(q_dtype);
-    default: return scaled_parts_q<BF16>(q_dtype);
   }
 }
 
@@ -1997,7 +1983,7 @@ extern "C" int grm_hip_retrieve_fuse(const void* memories, const int64_t* indice
       return GRM_HIP_EUNSUPPORTED;
     }
     const int64_t spread_tiles = tiles_max(segments, n_index, true);  // not more than the workspace holds
-    if (rows_in_lds(a, scaled_parts(mem_dtype, q_dtype), spread_tiles)) {
+    if (rows_in_lds(a, spread_tiles)) {
       a.lds_rows = 1;
       a.tile_pairs = static_cast<int>(tile_pairs_for(segments, n_index, true));
       a.tb_max = static_cast<int>(spread_tiles);

@@ -640,13 +640,14 @@ def test_retrieve_partial_steps(dev, pairs):
 @pytest.mark.parametrize("B,Q,S,R,H,K", [(1, 1, 3, 1, 8, 32), (1, 47, 1, 1, 32, 32), (2, 49, 2, 2, 64, 40),
                                          (1, 300, 1, 1, 128, 128), (1, 385, 1, 1, 128, 128),
                                          (2, 1700, 2, 2, 136, 120), (1, 5000, 5, 4, 512, 64), (1, 9000, 3, 8, 72, 16),
-                                         (1, 1, 3, 2, 40, 72), (2, 1, 2, 1, 64, 88)])
+                                         (1, 1, 3, 2, 32, 72), (2, 1, 2, 1, 24, 88), (1, 1, 2, 1, 32, 128)])
 def test_retrieve_fuse_states_in_lds(dev, mem_dtype, q_dtype, B, Q, S, R, H, K):
     """retrieve_fuse where a state is kept in LDS for many pairs: fewer pairs than a wave takes,
     one more than one and than eight waves take (48, 384), value widths of every padded size with
-    partial tiles, key widths below the padded ones, a single query that ends before the last padded
-    key step begins, sorts over one workgroup and over several (65536 pairs on); states of very different magnitude, and pairs with
-    an invalid index whose gate is NaN (absent, whatever its gate).  Rows are kept as float16 scaled
+    partial tiles, key widths below the padded ones, a single query (one that ends before the last
+    padded key step begins takes the other kernel), sorts over one workgroup and over several (65536
+    pairs on); states of very different magnitude, and pairs with an invalid index whose gate is NaN
+    (absent, whatever its gate).  Rows are kept as float16 scaled
     by their largest value: 2^-11 of it each, R of them summed under gates that add to one, before
     a LayerNorm of unit scale, so 2e-3 of the output's largest value bounds the error."""
     g = torch.Generator().manual_seed(Q + H)
