@@ -126,15 +126,13 @@ int grm_hip_chunk_update_fwd_noalloc(const void* keys, const void* values, const
  * dkq_partial: float32 workspace [2, batch, ceil(value_dim / 16), seq_len, key_dim]
  *   (caller-provided).  Both forms of the backward keep an adjoint dL/dM per 64-token
  *   chunk, [batch, ceil(seq_len / 64), value_dim, key_dim], at its front (the MFMA kernels
- *   for 16-bit inputs run when that fits, from about ten tokens on; the float32 kernels
- *   need none for a single chunk).  The MFMA kernels' follow it, when the walk over the
+ *   for 16-bit inputs run when that fits, from eight tokens on; the float32 kernels
+ *   need none for a single chunk, and for a few tokens only the partial sums).  The MFMA kernels' follow it, when the walk over the
  *   chunks runs in parts, by each part's adjoint at its start
  *   [batch, parts, value_dim, key_dim]; the float32 kernels', when several workgroups
  *   share a chunk, by their partial sums of grad_keys and grad_queries.
  * For float32 inputs a gradient may take the place of the tensor it belongs to, and
- * grad_memory that of grad_memory_out (with fewer than 8 tokens not grad_memory and the
- * others at once: refused where it does not work).  For 16-bit inputs no output may
- * overlap an input.
+ * grad_memory that of grad_memory_out.  For 16-bit inputs no output may overlap an input.
  * Infinities and NaN: with float32 inputs, and no gradient over values or grad_hidden, a
  * token's reach only the gradients that depend on it; otherwise also others of its block
  * of 16 tokens.

@@ -827,7 +827,7 @@ extern "C" int grm_hip_chunk_update_bwd(const void* grad_hidden, const void* gra
   const char* env = getenv("GRM_HIP_BWD_MFMA");
   // The MFMA kernels keep the adjoint at every chunk end, [batch, n_chunks,
   // value_dim, key_dim] float32, in dkq_partial: used where that fits the
-  // buffer's documented size (from about ten tokens on; shorter sequences take
+  // buffer's documented size (from eight tokens on; shorter sequences take
   // the float32 kernels, which need none for a single chunk).
   const bool gbuf_fits = n_chunks * value_dim <= 2 * tiles * seq_len;
   const bool mfma = (env == nullptr || env[0] != '0') && (in_dtype == GRM_HIP_BF16 || in_dtype == GRM_HIP_F16) &&

@@ -20,6 +20,7 @@
 //                     of the value tiles), on float32 MFMA
 // With few chunks the value tiles of one chunk are shared by several workgroups
 // (`splits`), whose dQ and dK are partial sums that split_sum_kernel adds in order.
+// A handful of tokens goes one by one instead (bwd_tokens_kernel, few_tokens).
 //
 // What bounds it: float32 MFMA (16x16x4, 256 FLOP per CU and clock).  Every
 // operand comes from LDS as 16 bytes of a row or as four single elements of a
@@ -168,6 +169,114 @@ template <class E>
 __global__ __launch_bounds__(GNT) void bwd_state_copy_kernel(const float* from, void* to, int64_t n, int f32) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * GNT + threadIdx.x;
   if (i < n) st_state<E>(to, i, f32 != 0, from[i]);
+}
+
+// A few tokens, one by one.  One wave per sequence and 16 value rows, lanes hold the key
+// columns in steps of 64: forward over the tokens for M_t and dQ, backward for G_t, dK and
+// dV (a reduction over the keys by a 16-value transposing butterfly, 17 shuffles per
+// token).  dQ and dK of the 16 rows are partial sums, [batch, value tiles, T, dk].  Bound by
+// the latency of each token's loads.
+constexpr int TOK_ROWS = 16;
+template <class E, int KR>
+__global__ __launch_bounds__(64) void bwd_tokens_kernel(const BwdGenArgs a) {
+  using raw = typename ET<E>::raw;
+  constexpr int RB = TOK_ROWS;
+  const int lane = threadIdx.x;
+  const int64_t b = blockIdx.x / static_cast<unsigned>(a.splits);
+  const int tile = static_cast<int>(blockIdx.x % static_cast<unsigned>(a.splits));
+  const int v0 = tile * RB;
+  const int dk = a.dk, dv = a.dv, T = static_cast<int>(a.T);
+  const float lam = a.pw[1], c = a.c;
+  const bool f32m = a.mem_f32 != 0;
+  const raw* keys = static_cast<const raw*>(a.keys) + b * T * dk;
+  const raw* queries = static_cast<const raw*>(a.queries) + b * T * dk;
+  const raw* values = static_cast<const raw*>(a.values) + b * T * dv;
+  const raw* dhp = static_cast<const raw*>(a.dh) + b * T * dv;
+  const int64_t part = (b * a.splits + tile) * static_cast<int64_t>(T) * dk;
+  float M[RB][KR], G[RB][KR];
+#pragma unroll
+  for (int r = 0; r < RB; ++r)
+#pragma unroll
+    for (int e = 0; e < KR; ++e) {
+      const int v = v0 + r, k = lane + 64 * e;
+      const bool in = v < dv && k < dk;
+      const int64_t i = (b * dv + v) * dk + k;
+      M[r][e] = in ? ld_state<E>(a.memory, i, f32m) : 0.f;
+      G[r][e] = in ? ld_state<E>(a.dmo, i, f32m) : 0.f;
+    }
+  for (int t = 0; t < T; ++t) {
+    float kt[KR], dq[KR];
+#pragma unroll
+    for (int e = 0; e < KR; ++e) {
+      const int k = lane + 64 * e;
+      kt[e] = k < dk ? ET<E>::to_f(keys[t * dk + k]) : 0.f;
+      dq[e] = 0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const int v = v0 + r;
+      const float cv = c * (v < dv ? ET<E>::to_f(values[static_cast<int64_t>(t) * dv + v]) : 0.f);
+      const float dh = v < dv ? ET<E>::to_f(dhp[static_cast<int64_t>(t) * dv + v]) : 0.f;
+#pragma unroll
+      for (int e = 0; e < KR; ++e) {
+        M[r][e] = fmaf(M[r][e], lam, cv * kt[e]);
+        dq[e] = fmaf(dh, M[r][e], dq[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < KR; ++e)
+      if (lane + 64 * e < dk) a.part_q[part + t * dk + lane + 64 * e] = dq[e];
+  }
+  for (int t = T - 1; t >= 0; --t) {
+    float kt[KR], qt[KR], dkt[KR], dvp[RB];
+#pragma unroll
+    for (int e = 0; e < KR; ++e) {
+      const int k = lane + 64 * e;
+      kt[e] = k < dk ? ET<E>::to_f(keys[t * dk + k]) : 0.f;
+      qt[e] = k < dk ? ET<E>::to_f(queries[t * dk + k]) : 0.f;
+      dkt[e] = 0.f;
+    }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const int v = v0 + r;
+      const float vv = v < dv ? ET<E>::to_f(values[static_cast<int64_t>(t) * dv + v]) : 0.f;
+      const float dh = v < dv ? ET<E>::to_f(dhp[static_cast<int64_t>(t) * dv + v]) : 0.f;
+      dvp[r] = 0.f;
+#pragma unroll
+      for (int e = 0; e < KR; ++e) {
+        G[r][e] = fmaf(dh, qt[e], t == T - 1 ? G[r][e] : G[r][e] * lam);
+        dkt[e] = fmaf(G[r][e], vv, dkt[e]);
+        dvp[r] = fmaf(G[r][e], kt[e], dvp[r]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < KR; ++e)
+      if (lane + 64 * e < dk) a.part_k[part + t * dk + lane + 64 * e] = c * dkt[e];
+    // 16 row sums over 64 lanes: halve the value count per exchange.
+#pragma unroll
+    for (int half = RB / 2, d = 32; half >= 1; half >>= 1, d >>= 1) {
+      const bool up = (lane & d) != 0;
+#pragma unroll
+      for (int i = 0; i < half; ++i) {
+        const float send = up ? dvp[i] : dvp[i + half];
+        const float keep = up ? dvp[i + half] : dvp[i];
+        dvp[i] = keep + __shfl_xor(send, d, 64);
+      }
+    }
+    float tot = dvp[0];
+    tot += __shfl_xor(tot, 2, 64);
+    tot += __shfl_xor(tot, 1, 64);
+    const int v = v0 + ((lane >> 5) & 1) * 8 + ((lane >> 4) & 1) * 4 + ((lane >> 3) & 1) * 2 + ((lane >> 2) & 1);
+    if ((lane & 3) == 0 && v < dv)
+      static_cast<raw*>(a.dv_out)[(b * T + t) * dv + v] = ET<E>::from_f(c * tot);
+  }
+#pragma unroll
+  for (int r = 0; r < RB; ++r)
+#pragma unroll
+    for (int e = 0; e < KR; ++e) {
+      const int v = v0 + r, k = lane + 64 * e;
+      if (v < dv && k < dk) st_state<E>(a.dm_out, (b * dv + v) * dk + k, f32m, G[r][e] * lam);
+    }
 }
 
 template <class E, int DKP>
@@ -537,10 +646,17 @@ __global__ __launch_bounds__(GNT) void split_sum_kernel(const BwdGenArgs a) {
   }
 }
 
+template <class E>
+int launch_split_sum(const BwdGenArgs& a, hipStream_t s) {
+  const int64_t want = (a.batch * a.T * a.dk + GNT - 1) / GNT;
+  hipLaunchKernelGGL(split_sum_kernel<E>, dim3(static_cast<unsigned>(std::min<int64_t>(want, 4096)), 2), dim3(GNT), 0,
+                     s, a);
+  return check_launch("chunk_update_bwd(split sum)");
+}
+
 // copy_to: grad_memory where a.dm_out is scratch, else NULL.
-// outer_last (one chunk): the kernel that writes grad_memory runs after the other.
 template <class E, int DKP>
-int launch_gen(const BwdGenArgs& a, void* copy_to, bool outer_last, hipStream_t s) {
+int launch_gen(const BwdGenArgs& a, void* copy_to, hipStream_t s) {
   using S = GenShape<E, DKP>;
   if (S::lds_bytes > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_chunk_kernel<E, DKP>),
@@ -554,12 +670,9 @@ int launch_gen(const BwdGenArgs& a, void* copy_to, bool outer_last, hipStream_t 
   const int64_t bc = a.batch * a.n_chunks;
   const int64_t n = a.batch * a.dv * a.dk;
   const dim3 state_grid(static_cast<unsigned>((n + GNT - 1) / GNT));
-  auto outer = [&] {
-    hipLaunchKernelGGL((bwd_outer_kernel<E, DKP>), dim3(static_cast<unsigned>(bc * ((a.dv + OUTER_V - 1) / OUTER_V))),
-                       dim3(GNT), 0, s, a);
-    return check_launch("chunk_update_bwd(outer)");
-  };
-  int rc = outer_last ? GRM_HIP_OK : outer();
+  hipLaunchKernelGGL((bwd_outer_kernel<E, DKP>), dim3(static_cast<unsigned>(bc * ((a.dv + OUTER_V - 1) / OUTER_V))),
+                     dim3(GNT), 0, s, a);
+  int rc = check_launch("chunk_update_bwd(outer)");
   if (rc != GRM_HIP_OK) return rc;
   if (a.n_chunks > 1) {
     hipLaunchKernelGGL(bwd_carry_kernel<E>, state_grid, dim3(GNT), 0, s, a);
@@ -570,68 +683,95 @@ int launch_gen(const BwdGenArgs& a, void* copy_to, bool outer_last, hipStream_t 
                      a);
   rc = check_launch("chunk_update_bwd(gradients)");
   if (rc != GRM_HIP_OK) return rc;
-  if (outer_last) rc = outer();
-  if (rc != GRM_HIP_OK) return rc;
   if (copy_to != nullptr) {
     hipLaunchKernelGGL(bwd_state_copy_kernel<E>, state_grid, dim3(GNT), 0, s, static_cast<const float*>(a.dm_out),
                        copy_to, n, a.mem_f32);
     rc = check_launch("chunk_update_bwd(state copy)");
     if (rc != GRM_HIP_OK) return rc;
   }
-  if (a.splits == 1) return rc;
-  const int64_t want = (a.batch * a.T * a.dk + GNT - 1) / GNT;
-  hipLaunchKernelGGL(split_sum_kernel<E>, dim3(static_cast<unsigned>(std::min<int64_t>(want, 4096)), 2), dim3(GNT), 0,
-                     s, a);
-  return check_launch("chunk_update_bwd(split sum)");
+  return a.splits == 1 ? rc : launch_split_sum<E>(a, s);
 }
 
 template <class E>
-int launch_gen_width(const BwdGenArgs& a, void* copy_to, bool outer_last, hipStream_t s) {
-  if (a.dk <= 32) return launch_gen<E, 32>(a, copy_to, outer_last, s);
-  if (a.dk <= 64) return launch_gen<E, 64>(a, copy_to, outer_last, s);
-  if (a.dk <= 128) return launch_gen<E, 128>(a, copy_to, outer_last, s);
-  if constexpr (sizeof(typename ET<E>::raw) == 2) return launch_gen<E, 256>(a, copy_to, outer_last, s);
+int launch_tokens(const BwdGenArgs& a, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(a.batch * a.splits));
+  if (a.dk <= 64) hipLaunchKernelGGL((bwd_tokens_kernel<E, 1>), grid, dim3(64), 0, s, a);
+  else if (std::is_same_v<E, F32> || a.dk <= 128)
+    hipLaunchKernelGGL((bwd_tokens_kernel<E, 2>), grid, dim3(64), 0, s, a);
+  else if constexpr (!std::is_same_v<E, F32>)
+    hipLaunchKernelGGL((bwd_tokens_kernel<E, 4>), grid, dim3(64), 0, s, a);
+  const int rc = check_launch("chunk_update_bwd(tokens)");
+  return rc != GRM_HIP_OK ? rc : launch_split_sum<E>(a, s);
+}
+
+template <class E>
+int launch_gen_width(const BwdGenArgs& a, void* copy_to, hipStream_t s) {
+  if (a.dk <= 32) return launch_gen<E, 32>(a, copy_to, s);
+  if (a.dk <= 64) return launch_gen<E, 64>(a, copy_to, s);
+  if (a.dk <= 128) return launch_gen<E, 128>(a, copy_to, s);
+  if constexpr (sizeof(typename ET<E>::raw) == 2) return launch_gen<E, 256>(a, copy_to, s);
   set_error("chunk_update_bwd: key_dim %d exceeds 128 for float32", a.dk);
   return GRM_HIP_EUNSUPPORTED;
+}
+
+// Workgroups of one chunk's value tiles: enough for two per CU, at least two tiles each
+// (a split repeats the chunk's P and its dS products, worth about one tile's work).
+int64_t splits_for(int64_t chunks, int64_t vtiles) {
+  return std::max<int64_t>(1, std::min<int64_t>((512 + chunks - 1) / chunks, vtiles / 2));
+}
+
+// Token by token where a 64-token chunk is mostly padding: it costs its 20 to 80 us
+// whatever T, a token 5 (float32) to 10 us.  Whole call, chunk kernels and token kernel, us:
+//   key_dim 64, value_dim 64, 16 sequences, float32: 2 tokens 26 and 22, 3 tokens 26 and 24,
+//     4 tokens 26 and 28; float16: 29 and 26, 28 and 34
+//   (128, 128), 16 sequences, float32: 1 token 44 and 21, 5 tokens 44 and 40, 6 tokens 44
+//     and 45; float16: 3 tokens 47 and 40, 4 tokens 48 and 49; key_dim 200, 5 tokens 82 and 68
+//   (128, 128), 256 sequences (more workgroups than the one per CU that its LDS allows),
+//     float32: 8 tokens 78 and 67, 12 tokens 79 and 108; float16: 4 tokens 82 and 60
+//   up to 32 keys the chunk kernels are at the host's 21 us for any of these
+// It also takes the short calls that have no room for grad_memory in scratch.
+bool few_tokens(const BwdGenArgs& a, int in_dtype, bool in_place) {
+  const bool f32 = in_dtype == GRM_HIP_F32;
+  const bool full = a.batch * splits_for(a.batch, (a.dv + kGenDv - 1) / kGenDv) > 256;
+  const int most = a.dk <= 32    ? 0
+                   : a.dk <= 64  ? (f32 ? 3 : 2)
+                   : a.dk <= 128 ? (f32 ? (full ? 8 : 5) : (full ? 4 : 3))
+                                 : 5;
+  return a.T <= most || (in_place && a.T < 8);
 }
 
 }  // namespace
 
 int launch_bwd_gen(BwdGenArgs a, int in_dtype, float* ws, int64_t floats, hipStream_t s) {
-  const int64_t vtiles = (a.dv + kGenDv - 1) / kGenDv;
-  const int64_t state = a.batch * static_cast<int64_t>(a.dv) * a.dk;
-  int64_t adj = a.n_chunks > 1 ? a.n_chunks * state : 0;
-  // grad_memory in the place of grad_memory_out or memory, which bwd_chunk_kernel reads: it
-  // goes through scratch behind the adjoints.  From eight tokens on the documented workspace
-  // has room for that; below, grad_memory is written last, from rows that must still be there.
-  const int64_t es = in_dtype == GRM_HIP_F32 ? 4 : 2, state_b = state * (a.mem_f32 != 0 ? 4 : 2);
-  const int64_t kb = a.batch * a.T * a.dk * es, vb = a.batch * a.T * a.dv * es;
-  const void* const outs[] = {a.dq_out, a.dk_out, a.dv_out};
-  const int64_t out_b[] = {kb, kb, vb};
+  const int64_t state = a.batch * static_cast<int64_t>(a.dv) * a.dk, state_b = state * (a.mem_f32 != 0 ? 4 : 2);
   const bool in_place =
       ranges_overlap(a.dm_out, state_b, a.dmo, state_b) || ranges_overlap(a.dm_out, state_b, a.memory, state_b);
-  void* copy_to = nullptr;
-  bool outer_last = false;
+  const int64_t rows = a.batch * a.T * a.dk;
   a.dm_f32 = a.mem_f32;
+  if (few_tokens(a, in_dtype, in_place)) {
+    a.splits = (a.dv + TOK_ROWS - 1) / TOK_ROWS;
+    a.part_k = ws;
+    a.part_q = ws + a.splits * rows;
+    switch (in_dtype) {
+      case GRM_HIP_F32: return launch_tokens<F32>(a, s);
+      case GRM_HIP_F16: return launch_tokens<F16>(a, s);
+      default: return launch_tokens<BF16>(a, s);
+    }
+  }
+  const int64_t vtiles = (a.dv + kGenDv - 1) / kGenDv;
+  int64_t adj = a.n_chunks > 1 ? a.n_chunks * state : 0;
+  // grad_memory in the place of grad_memory_out or memory, which bwd_chunk_kernel reads: it
+  // goes through scratch behind the adjoints, for which the documented workspace has room
+  // from eight tokens on.
+  void* copy_to = nullptr;
   if (in_place && adj + state <= floats) {
     copy_to = a.dm_out;
     a.dm_out = ws + adj;
     a.dm_f32 = 1;
     adj += state;
-  } else if (in_place) {
-    outer_last = true;
-    for (int o = 0; o < 3; ++o)
-      if (ranges_overlap(outs[o], out_b[o], a.queries, kb) || ranges_overlap(outs[o], out_b[o], a.dh, vb)) {
-        set_error("chunk_update_bwd: fewer than 8 tokens with grad_memory and the rows' gradients in place");
-        return GRM_HIP_EINVAL;
-      }
   }
-  // Enough workgroups for two per CU, at least two value tiles each (a split
-  // repeats the chunk's P and its dS products, worth about one tile's work), and
-  // the partial sums within the workspace.
   const int64_t bc = a.batch * a.n_chunks;
-  int64_t splits = std::max<int64_t>(1, std::min<int64_t>((512 + bc - 1) / bc, vtiles / 2));
-  const int64_t rows = a.batch * a.T * a.dk;
+  int64_t splits = splits_for(bc, vtiles);  // fewer where their partial sums exceed the workspace
   while (splits > 1 && adj + 2 * splits * rows > floats) --splits;
   const int64_t per = (vtiles + splits - 1) / splits;
   a.tiles_per_split = static_cast<int>(per);
@@ -643,15 +783,18 @@ int launch_bwd_gen(BwdGenArgs a, int in_dtype, float* ws, int64_t floats, hipStr
   }
   // bwd_chunk_kernel may read values and grad_hidden again after it has written gradients.
   a.exact = static_cast<int64_t>(a.dv) * a.dk * 4 <= INT32_MAX;
+  const int64_t es = in_dtype == GRM_HIP_F32 ? 4 : 2, kb = rows * es, vb = a.batch * a.T * a.dv * es;
+  const void* const outs[] = {a.dq_out, a.dk_out, a.dv_out};
+  const int64_t out_b[] = {kb, kb, vb};
   for (int o = 0; o < 3; ++o)
     if (ranges_overlap(outs[o], out_b[o], a.values, vb) || ranges_overlap(outs[o], out_b[o], a.dh, vb)) a.exact = 0;
   a.gbuf = ws;
   a.part_k = ws + adj;
   a.part_q = ws + adj + a.splits * rows;
   switch (in_dtype) {
-    case GRM_HIP_F32: return launch_gen_width<F32>(a, copy_to, outer_last, s);
-    case GRM_HIP_F16: return launch_gen_width<F16>(a, copy_to, outer_last, s);
-    default: return launch_gen_width<BF16>(a, copy_to, outer_last, s);
+    case GRM_HIP_F32: return launch_gen_width<F32>(a, copy_to, s);
+    case GRM_HIP_F16: return launch_gen_width<F16>(a, copy_to, s);
+    default: return launch_gen_width<BF16>(a, copy_to, s);
   }
 }
 
