@@ -721,10 +721,13 @@ int launch_bwd_mfma(BwdMArgs a, int mem_dtype, hipStream_t s) {
   static_assert(AjShape<DKP, 4>::lds_bytes <= 64 * 1024, "no attribute needed");
   int rc = allow_lds(&bwd_grad_kernel<E, DKP>, GrShape<DKP>::lds_bytes, attr_g);
   if (rc != GRM_HIP_OK) return rc;
-  // 32-row workgroups where 64-row ones would leave CUs idle: each walks the same
-  // chunks with half the work per step (64 x 2048 tokens of width 128, 128 -> 256
-  // workgroups, 68 -> 61 us).
-  const bool narrow = a.batch * ((a.dv + AJ_V - 1) / AJ_V) * a.n_parts < 192;
+  // 32-row workgroups where they are no more than the CUs: each walks the same chunks
+  // with half the work per step (64 x 2048 tokens of width 128, 128 -> 256 workgroups,
+  // 68 -> 61 us; whole backwards of 300 to 2048 tokens 1.03 to 1.08 times as fast).
+  // With more of them some CUs have two: 150 to 191 sequences of 64 values, 300 to 2048
+  // tokens, took 1.03 to 1.09 times as long (180 x 2048, key width 64, 156 -> 172 us).
+  const int64_t narrow_grid = a.batch * ((a.dv + AJ_V / 2 - 1) / (AJ_V / 2)) * a.n_parts;
+  const bool narrow = narrow_grid <= 256;
   const int rows = narrow ? AJ_V / 2 : AJ_V;
   const int64_t grid_a = a.batch * ((a.dv + rows - 1) / rows) * a.n_parts;
   a.xcd_remap = (grid_a % 8 == 0) ? 1 : 0;

@@ -389,7 +389,7 @@ def close_elementwise(name, got, ref, rtol=2e-2, atol=2e-3):
                                              (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16)])
 @pytest.mark.parametrize("B,T,K,H", [(2, 300, 128, 128), (3, 129, 64, 64), (1, 640, 96, 96), (2, 64, 128, 32),
                                      (1, 7, 128, 32), (1, 12, 128, 32), (2, 200, 32, 64), (1, 200, 64, 512),
-                                     (1, 2000, 64, 512), (2, 1000, 64, 96), (96, 70, 128, 96), (200, 70, 64, 32)])
+                                     (1, 2000, 64, 512), (2, 1000, 64, 96), (96, 70, 128, 96), (300, 70, 64, 32)])
 def test_mfma_backward(dev, monkeypatch, dtype, mem_dtype, B, T, K, H):
     """The chunk-parallel MFMA backward (16-bit inputs, value_dim a multiple of 32: the adjoint
     pass, then the per-chunk gradients over every value tile) against the double-precision
@@ -398,8 +398,8 @@ def test_mfma_backward(dev, monkeypatch, dtype, mem_dtype, B, T, K, H):
     sixteen value tiles, one chunk (12 tokens), 7 tokens, where the adjoint buffer would not
     fit the workspace and the float32 kernels run, and adjoint walks split into 2, 4 and 8
     parts (640, 1000 and 2000 tokens).  All of these walk 32 value rows per workgroup; the
-    two with 192 and 200 workgroups of 64 rows walk those, with half-filled ones (96 and 32
-    values), in one part that writes grad_memory itself."""
+    two with more than 256 such workgroups (96 and 300 sequences) walk 64, with half-filled
+    workgroups (96 and 32 values), in one part that writes grad_memory itself."""
     k, v, q, m = make_case(B, T, K, H, dtype, mem_dtype, seed=B * 13 + T)
     g = torch.Generator().manual_seed(7)
     dh = torch.randn(B, T, H, generator=g).to(dtype)
