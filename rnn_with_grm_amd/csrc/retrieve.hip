@@ -452,7 +452,10 @@ __global__ __launch_bounds__(AP_THREADS) void apply_bucket_kernel(const Retrieve
         const int p = e / DKP, k = e % DKP;
         const int pid = pair_id[p];
         float x = 0.f;
-        if (pid >= 0 && k < dk) x = ET<EM>::to_f(ET<EM>::from_f(ET<EQ>::to_f(qsrc[static_cast<int64_t>(query_of(a, pid)) * dk + k])));
+        if (pid >= 0 && k < dk) {
+          const rawq q = qsrc[static_cast<int64_t>(query_of(a, pid)) * dk + k];
+          x = ET<EM>::to_f(ET<EM>::from_f(ET<EQ>::to_f(q)));
+        }
         QO[p * QS + k] = x;
       }
     }
@@ -1072,7 +1075,7 @@ namespace {
 // That kernel holds 32 rows per wave and passes every 64-pair output tile through
 // LDS with two barriers and eight dependent scale-and-store rounds per wave, which
 // cost more than its memory traffic.  16 x 65536 queries, 16 of 512 states of
-// 128 x 128: 3.4 ms there, 2.33 ms here (2.20 without the scattered 4-byte read of
+// 128 x 128: 3.4 ms there, 2.29 ms here (2.20 without the scattered 4-byte read of
 // each pair's gate).  What bounds it now: the 256-byte query rows read and the rows
 // written, both scattered, about 11 GB through the L2 misses at 4.7 TB/s (a 1 GiB copy
 // reaches 5.2); without the row stores 1.0 ms less, with 32 or 64 pairs per wave and
@@ -1110,7 +1113,8 @@ __global__ __launch_bounds__(AL_THREADS, 2) void apply_lds_kernel(const Retrieve
   const __amdgpu_buffer_rsrc_t rscale =
       make_rsrc(a.scales + b * a.n_index * a.v_tiles, static_cast<uint32_t>(a.n_index * a.v_tiles * 4));
   auto load_id = [&](int p) {  // -1 past the tile
-    const int id = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rl, p + lane < p_end ? (p + lane) * 4 : kBufOOB, 0, 0));
+    const int off = p + lane < p_end ? (p + lane) * 4 : kBufOOB;
+    const int id = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rl, off, 0, 0));
     return p + lane < p_end ? id : -1;
   };
 

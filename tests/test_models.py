@@ -441,7 +441,7 @@ def _bf16_training_grads(dev, dtype):
 @pytest.mark.gpu
 def test_training_gradients_bf16_mfma_backward(dev, monkeypatch):
     """bf16 training through the MFMA scan backward: every parameter gradient against the
-    same bf16 model with the per-token float32 backward kernel (GRM_HIP_BWD_MFMA=0; the two
+    same bf16 model with the float32-arithmetic backward (GRM_HIP_BWD_MFMA=0; the two
     runs differ only in the scan's backward) and against the float32 model (which also
     differs by bf16 rounding of every activation), as relative L2 error per parameter.  The
     float32 bar is looser for the routing projections, whose gradients pass through a
@@ -450,19 +450,19 @@ def test_training_gradients_bf16_mfma_backward(dev, monkeypatch):
     print(f"bf16 training gradients, MFMA backward, on {dev}", flush=True)
     mfma = _bf16_training_grads(dev, torch.bfloat16)
     monkeypatch.setenv("GRM_HIP_BWD_MFMA", "0")
-    scalar = _bf16_training_grads(dev, torch.bfloat16)
+    f32_bwd = _bf16_training_grads(dev, torch.bfloat16)
     monkeypatch.delenv("GRM_HIP_BWD_MFMA")
     ref = _bf16_training_grads(dev, torch.float32)
-    assert mfma.keys() == scalar.keys() == ref.keys() and len(mfma) > 10
+    assert mfma.keys() == f32_bwd.keys() == ref.keys() and len(mfma) > 10
     worst_kernel, worst_f32, worst_cell = 0.0, 0.0, 0.0
     for name, r in ref.items():
         den = float(r.norm())
         if den == 0.0:
             assert float(mfma[name].norm()) == 0.0, name
             continue
-        rel_kernel = float((mfma[name] - scalar[name]).norm()) / max(float(scalar[name].norm()), 1e-30)
+        rel_kernel = float((mfma[name] - f32_bwd[name]).norm()) / max(float(f32_bwd[name].norm()), 1e-30)
         rel_f32 = float((mfma[name] - r).norm()) / den
-        print(f"  {name}: vs per-token kernel {rel_kernel:.2e}, vs float32 {rel_f32:.2e}", flush=True)
+        print(f"  {name}: vs float32 kernels {rel_kernel:.2e}, vs float32 {rel_f32:.2e}", flush=True)
         worst_kernel, worst_f32 = max(worst_kernel, rel_kernel), max(worst_f32, rel_f32)
         if "memory_cell" in name:
             worst_cell = max(worst_cell, rel_f32)
